@@ -102,9 +102,12 @@ int64_t decode_fused_units(int64_t n_head, int64_t n_kv_head);
 size_t decode_fused_partial_bytes(int64_t batch, int64_t n_head, int64_t n_kv_head,
                                   int64_t t_max, int64_t window);
 
-// The general chunked prefill (any dtype, head_dim up to 512); it also serves single-token
-// calls with head_dim above 256, past what the split-K decode kernel takes.
+// Attention at head_dim above 256, up to 512 (any dtype): chunked prefill, and single-token calls,
+// past what the split-K decode kernel takes.
 int launch_prefill_generic(const AttnArgs &a);
+
+// The chunked prefill on the matrix cores for fp32 caches and other head dims up to 256.
+int launch_prefill_tiled(const AttnArgs &a);
 
 // The bf16 / head_dim 128 chunked prefill on the matrix cores.
 bool prefill_mfma_supported(const AttnArgs &a);

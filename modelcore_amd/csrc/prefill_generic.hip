@@ -1,17 +1,19 @@
-// Multi-token attention against the cache prefix, any head_dim up to 256 made of whole 16-byte
-// vectors, bf16 or fp32.
+// Attention against the cache prefix for head dims above 256 (up to 512, made of whole 16-byte
+// vectors), bf16 or fp32: multi-token calls, and single-token ones, which the split-K decode kernel
+// takes up to 256 only.
 //
 // Semantics: modelcore/kernels/flash_attn.py:226-244 (uniform, explicit mask with row offset
 // Tk - Tq) and :362-364 (ragged mask). Query t of row b sits at p = cache_seqlens[b] + t and
 // attends keys col <= p with p - col <= window when window >= 0. The cache already holds the new
 // tokens (the append runs first), so the prefix includes the chunk itself.
 //
-// This is the general-shape kernel (fp32 caches, small or odd head counts and head dims); the bf16
-// MFMA kernel in prefill_mfma.hip takes the large shapes. One workgroup owns 64 (query, head)
+// Smaller heads run on the matrix cores (prefill_mfma.hip, prefill_tiled.hip).
+//
+// One workgroup owns 64 (query, head)
 // rows of one KV head: 64 / G consecutive queries times the G query heads that share the KV head,
 // so every K/V tile staged in LDS serves all of them. Four lanes share a row, each owning every
 // fourth dimension (of the head_dim rounded up to a power of two; dims past the real head_dim
-// stay zero). Keys are walked in tiles of 32 from the first key any row of the block can see to
+// stay zero). Keys are walked in tiles of 16 from the first key any row of the block can see to
 // the last; each tile's scores are masked per row, and an online softmax (running max m,
 // running sum l, rescaled accumulator) folds the tile in.
 #include "kernels.h"
@@ -23,9 +25,8 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRows = 64;
-// Keys per LDS tile: 32, or 16 for head dims above 256 (K and V tiles of 64 KiB in fp32).
-template <int DP>
-constexpr int kTileKeys = DP <= 256 ? 32 : 16;
+constexpr int DP = 512;         // head_dim rounded up
+constexpr int kTileKeys = 16;   // keys per LDS tile (K and V tiles of 32 KiB in fp32)
 
 struct PrefillParams {
   const void *q, *k_cache, *v_cache;
@@ -37,10 +38,10 @@ struct PrefillParams {
   float scale_log2;
 };
 
-template <class E, int DP>
+template <class E>
 __global__ __launch_bounds__(kThreads) void prefill_generic_kernel(PrefillParams P) {
   constexpr int DS = DP / 4;  // dimensions per lane (lane j owns d = 4*i + j, d < DP)
-  constexpr int KT = kTileKeys<DP>;
+  constexpr int KT = kTileKeys;
   constexpr int VEC = Vec<E>::N;
   const int D = P.D;          // the real head_dim (<= DP); dims past it are zero in LDS and q
   __shared__ float sk[KT][DP];
@@ -165,25 +166,11 @@ __global__ __launch_bounds__(kThreads) void prefill_generic_kernel(PrefillParams
   }
 }
 
-template <class E, int DP>
+template <class E>
 int run_prefill(const PrefillParams &P, int B, hipStream_t stream) {
   dim3 grid((P.T_new + P.QT - 1) / P.QT, P.H_kv, B);
-  hipLaunchKernelGGL((prefill_generic_kernel<E, DP>), grid, dim3(kThreads), 0, stream, P);
+  hipLaunchKernelGGL(prefill_generic_kernel<E>, grid, dim3(kThreads), 0, stream, P);
   return launch_status("prefill_generic");
-}
-
-template <class E>
-int dispatch_d(const PrefillParams &P, int D, int B, hipStream_t s) {
-  switch (head_dim_bucket(D)) {
-    case 16: return run_prefill<E, 16>(P, B, s);
-    case 32: return run_prefill<E, 32>(P, B, s);
-    case 64: return run_prefill<E, 64>(P, B, s);
-    case 128: return run_prefill<E, 128>(P, B, s);
-    case 256: return run_prefill<E, 256>(P, B, s);
-    case 512: return run_prefill<E, 512>(P, B, s);
-    default:
-      return fail(MCAMD_EUNSUPPORTED, "attention: head_dim must be at most 512");
-  }
 }
 
 }  // namespace
@@ -208,8 +195,8 @@ int launch_prefill_generic(const AttnArgs &a) {
   P.cache_b = a.cache_batch_stride;
   P.D = int(a.head_dim);
   P.scale_log2 = float(kLog2e / std::sqrt(double(a.head_dim)));
-  if (a.dtype == MCAMD_BF16) return dispatch_d<bf16>(P, int(a.head_dim), int(a.batch), a.stream);
-  return dispatch_d<float>(P, int(a.head_dim), int(a.batch), a.stream);
+  if (a.dtype == MCAMD_BF16) return run_prefill<bf16>(P, int(a.batch), a.stream);
+  return run_prefill<float>(P, int(a.batch), a.stream);
 }
 
 int launch_prefill(const AttnArgs &a) {
@@ -221,6 +208,7 @@ int launch_prefill(const AttnArgs &a) {
     return MCAMD_OK;
   }
   if (prefill_mfma_supported(a)) return launch_prefill_mfma(a);
+  if (a.head_dim <= 256) return launch_prefill_tiled(a);
   return launch_prefill_generic(a);
 }
 
