@@ -290,21 +290,28 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
     f32x16 s[MK];
 #pragma unroll
     for (int mk = 0; mk < MK; ++mk) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) s[mk][e] = 0.f;
       const E *kp = &sK[(wk + 32 * mk + col) * KSTR + VEC * h];
+      // fp32: four interleaved chains of sums, added at the end: a quarter of one chain's rounding.
+      constexpr int NC = kBf16 ? 1 : 4;
+      f32x16 sc[NC];
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[j][e] = 0.f;
 #pragma unroll
       for (int i = 0; i < NQ; ++i) {
         const QF a = __builtin_bit_cast(
             QF, *reinterpret_cast<const uint4 *>(kp + (kBf16 ? 16 : 8) * i));
         if constexpr (kBf16) {
-          s[mk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[i], s[mk], 0, 0, 0);
+          sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[i], sc[0], 0, 0, 0);
         } else {
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            s[mk] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], qf[i][j], s[mk], 0, 0, 0);
+            sc[j % NC] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], qf[i][j], sc[j % NC], 0, 0, 0);
         }
       }
+      s[mk] = sc[0];
+      if constexpr (!kBf16) s[mk] = (sc[0] + sc[1]) + (sc[2] + sc[3]);
     }
     // Keys the pair may not see, in tiles that straddle the diagonal or the window's edge.
     if (k0 + KW - 1 > p_first || (P.window >= 0 && k0 < hi - P.window)) {
