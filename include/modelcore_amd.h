@@ -93,6 +93,16 @@ size_t mcamd_attn_workspace_bytes(int64_t batch, int64_t t_new, int64_t n_head,
                                   int64_t window);
 
 /*
+ * Bytes of scratch with which the operator runs these sizes best. t_new == 1: what
+ * mcamd_attn_workspace_bytes() gives. t_new > 1, where no workspace is needed: room for the fp32
+ * partials of a call with too few queries to fill the GPU, whose keys are then cut into ranges
+ * (another order of the same fp32 sums); without it, or with less, such a call runs uncut. 0 where
+ * none is of use.
+ */
+size_t mcamd_attn_scratch_bytes(int64_t batch, int64_t t_new, int64_t n_head, int64_t n_kv_head,
+                                int64_t head_dim, int64_t t_max, int64_t window, int dtype);
+
+/*
  * The cached-attention operator: optional append of (k, v) at cache_seqlens (k and v both
  * NULL = no append), then attention of q over the cache under the rules at the top of this
  * file. t_new == 1 runs split-K flash-decoding; t_new > 1 runs chunked prefill against the
@@ -154,7 +164,8 @@ int mcamd_flash_attn_with_kvcache_ex(const void *q, const void *k, const void *v
  * GPU: calls that overlap on one GPU race. Sizes whose decode partials need more scratch than that
  * (mcamd_attn_workspace_bytes() > MCAMD_NOALLOC_SCRATCH_BYTES) return MCAMD_EWORKSPACE. The
  * stream's device must be the current device. Otherwise identical to
- * mcamd_flash_attn_with_kvcache, with the same kernels and bit-identical results.
+ * mcamd_flash_attn_with_kvcache, with the same kernels and bit-identical results (for t_new > 1,
+ * to that call without a workspace).
  */
 #define MCAMD_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
 int mcamd_flash_attn_with_kvcache_noalloc(const void *q, const void *k, const void *v,

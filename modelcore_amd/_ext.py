@@ -39,6 +39,7 @@ SIGNATURES = {
     "mcamd_kv_replicate": (_int, [_ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i64, _i64, _i64,
                                   _i64, _i64, _i64, _int, _ptr]),
     "mcamd_attn_workspace_bytes": (_size, [_i64, _i64, _i64, _i64, _i64, _i64, _i64]),
+    "mcamd_attn_scratch_bytes": (_size, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _int]),
     "mcamd_flash_attn_with_kvcache": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64,
                                              _i64, _i64, _i64, _i64, _i64, _i64, _int, _int, _ptr,
                                              _size, _ptr]),

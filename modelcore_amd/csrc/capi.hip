@@ -72,6 +72,27 @@ extern "C" size_t mcamd_attn_workspace_bytes(int64_t batch, int64_t t_new, int64
          decode_prefix_bytes(batch, n_head, n_kv_head, head_dim, t_max, window);
 }
 
+extern "C" size_t mcamd_attn_scratch_bytes(int64_t batch, int64_t t_new, int64_t n_head,
+                                           int64_t n_kv_head, int64_t head_dim, int64_t t_max,
+                                           int64_t window, int dtype) {
+  if (t_new == 1)
+    return mcamd_attn_workspace_bytes(batch, t_new, n_head, n_kv_head, head_dim, t_max, window);
+  if (t_new < 1 || batch <= 0 || n_kv_head <= 0 || n_head < n_kv_head || head_dim <= 0 ||
+      head_dim > 256 || t_max <= 0 || t_max > (int64_t(1) << 30) || batch > 65535 ||
+      n_head > 65535)
+    return 0;
+  AttnArgs a{};
+  a.batch = batch;
+  a.t_new = t_new;
+  a.n_head = n_head;
+  a.n_kv_head = n_kv_head;
+  a.head_dim = head_dim;
+  a.t_max = t_max;
+  a.window = window;
+  a.dtype = dtype;
+  return prefill_scratch_bytes(a);
+}
+
 extern "C" int mcamd_decode_attention(const void *q, const void *k_cache, const void *v_cache,
                                       const int32_t *cache_seqlens, void *out, int64_t batch,
                                       int64_t n_head, int64_t n_kv_head, int64_t head_dim,

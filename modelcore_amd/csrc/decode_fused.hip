@@ -848,6 +848,8 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
                                 2 * lane) = pack_bf16(t0 * inv, t1 * inv);
 }
 
+}  // namespace
+
 // Number of compute units of the current device, queried once per device. Threads that race on
 // the first query each store the same value; the atomics make that well-defined.
 int device_cus() {
@@ -862,8 +864,6 @@ int device_cus() {
   }
   return n;
 }
-
-}  // namespace
 
 int64_t decode_fused_units(int64_t n_head, int64_t n_kv_head) {
   const int64_t G = n_head / n_kv_head;

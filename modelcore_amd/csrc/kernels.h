@@ -57,6 +57,13 @@ struct AttnArgs {
 int launch_decode(const AttnArgs &a);
 int launch_prefill(const AttnArgs &a);
 
+// Compute units of the current device (256 without one).
+int device_cus();
+
+// Scratch with which launch_prefill can cut the keys of a call with few query blocks into ranges
+// (prefill_split.h); 0 where it would not. Without it the call runs uncut.
+size_t prefill_scratch_bytes(const AttnArgs &a);
+
 // Split-K geometry of the decode path: keys per split and the number of splits a row can need.
 constexpr int kDecodeSplitLen = 256;
 int64_t decode_max_splits(int64_t t_max, int64_t window);
@@ -112,6 +119,13 @@ int launch_prefill_tiled(const AttnArgs &a);
 // The bf16 / head_dim 128 chunked prefill on the matrix cores.
 bool prefill_mfma_supported(const AttnArgs &a);
 int launch_prefill_mfma(const AttnArgs &a);
+// Key ranges of these calls (prefill_split.h), and the merge of their partials into the output;
+// careful: results that are not finite are redone key by key.
+struct SplitPlan;
+struct SplitGeo;
+SplitPlan prefill_mfma_plan(const AttnArgs &a);
+SplitPlan prefill_tiled_splits(const AttnArgs &a);
+int launch_prefill_combine(const AttnArgs &a, const SplitGeo &g, bool careful);
 
 // Shape checks shared by every attention entry point.
 int check_attn_shapes(const AttnArgs &a, bool need_workspace);

@@ -16,7 +16,7 @@
 // stay zero). Keys are walked in tiles of 16 from the first key any row of the block can see to
 // the last; each tile's scores are masked per row, and an online softmax (running max m,
 // running sum l, rescaled accumulator) folds the tile in.
-#include "kernels.h"
+#include "prefill_split.h"
 
 #include <cmath>
 
@@ -197,6 +197,11 @@ int launch_prefill_generic(const AttnArgs &a) {
   P.scale_log2 = float(kLog2e / std::sqrt(double(a.head_dim)));
   if (a.dtype == MCAMD_BF16) return run_prefill<bf16>(P, int(a.batch), a.stream);
   return run_prefill<float>(P, int(a.batch), a.stream);
+}
+
+size_t prefill_scratch_bytes(const AttnArgs &a) {
+  if (a.head_dim > 256 || a.t_new < 2) return 0;
+  return split_bytes(a, prefill_mfma_supported(a) ? prefill_mfma_plan(a) : prefill_tiled_splits(a));
 }
 
 int launch_prefill(const AttnArgs &a) {

@@ -54,7 +54,7 @@
 //
 // The shared prompt prefix of a decode step runs inside the fused decode kernel (prefix_mfma.h),
 // built from the same fragments and layouts.
-#include "kernels.h"
+#include "prefill_split.h"
 
 #include <cmath>
 #include <type_traits>
@@ -145,12 +145,16 @@ __device__ __forceinline__ float exp2_or_zero(float x) {
   return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x);
 }
 
-__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P) {
+// SPLIT: a workgroup per key range of a block (prefill_split.h).
+template <bool SPLIT>
+__device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const SplitGeo *S) {
   __shared__ __attribute__((aligned(1024))) uint16_t sK[4][TILE];
   __shared__ __attribute__((aligned(1024))) uint16_t sV[4][TILE];
 
   const int bh = blockIdx.x % P.n_bh;
-  const int qt = blockIdx.x / P.n_bh;
+  const int rest = blockIdx.x / P.n_bh;
+  const int part = SPLIT ? rest % S->n_split : 0;  // key range
+  const int qt = SPLIT ? rest / S->n_split : rest;
   const int b = bh / P.H_kv;  // sequence (a cache row, or one prompt of a varlen batch)
   const int kvh = bh - b * P.H_kv;
   const int q0 = qt * P.QT;
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P)
   const int head = live ? pr - (pr / P.G) * P.G : 0;
   uint16_t *out = P.out + ((tok0 + pos) * P.H + int64_t(kvh) * P.G + head) * D;
   if (!row_ok) {
-    if (live)
+    if (live && part == 0)
       for (int d = h * 64; d < h * 64 + 64; ++d) out[d] = 0x7fc0;
     return;
   }
@@ -197,8 +201,18 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P)
   const int p_abs = s0 + pos;
   const int p_first = s0 + q0;
   const int p_last = s0 + q_end - 1;
-  const int lo = P.window >= 0 ? max(0, p_first - P.window) : 0;
-  const int hi = p_last;
+  int lo = P.window >= 0 ? max(0, p_first - P.window) : 0;
+  int hi = p_last;
+  bool whole = true;
+  if constexpr (SPLIT) {  // this workgroup's range of the block's tiles
+    const int tiles = (hi - lo) / KT + 1;
+    const int ranges = block_splits(*S, s0, T_b, tiles);
+    if (part >= ranges) return;
+    whole = ranges == 1;
+    const int t0 = part * tiles / ranges, t1 = (part + 1) * tiles / ranges;
+    hi = min(hi, lo + t1 * KT - 1);
+    lo += t0 * KT;
+  }
 
   const int64_t tok = int64_t(P.H_kv) * D;
   const uint16_t *kbase = P.k_cache + int64_t(row) * P.cache_b + int64_t(kvh) * D;
@@ -497,6 +511,19 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P)
   const float lt = sum_halves(l);
   const float inv = 1.f / lt;
   if (!live) return;
+  if constexpr (SPLIT) {
+    if (!whole) {
+      const int64_t g = S->group(part, qt, bh, wave);
+#pragma unroll
+      for (int md = 0; md < 4; ++md)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<float4 *>(S->o(g, md, j, lane)) =
+              make_float4(o[md][4 * j], o[md][4 * j + 1], o[md][4 * j + 2], o[md][4 * j + 3]);
+      if (h == 0) *reinterpret_cast<float2 *>(S->ml(g, col)) = make_float2(m, lt);
+      return;
+    }
+  }
 #pragma unroll
   for (int md = 0; md < 4; ++md)
 #pragma unroll
@@ -513,6 +540,13 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P)
     }
 }
 
+__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P) {
+  prefill_mfma_body<false>(P, nullptr);
+}
+__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_split_kernel(MfmaParams P, SplitGeo S) {
+  prefill_mfma_body<true>(P, &S);
+}
+
 }  // namespace
 
 bool prefill_mfma_geometry_ok(int64_t n_head, int64_t n_kv_head, int64_t t_max) {
@@ -525,6 +559,18 @@ bool prefill_mfma_geometry_ok(int64_t n_head, int64_t n_kv_head, int64_t t_max) 
 bool prefill_mfma_supported(const AttnArgs &a) {
   return a.dtype == MCAMD_BF16 && a.head_dim == D &&
          prefill_mfma_geometry_ok(a.n_head, a.n_kv_head, a.t_max);
+}
+
+SplitPlan prefill_mfma_plan(const AttnArgs &a) {
+  const int64_t G = a.n_head / a.n_kv_head, QT = kPairs / G;
+  SplitPlan p;
+  p.pairs = int(QT * G);
+  p.kt = KT;
+  p.blocks = (a.t_new + QT - 1) / QT * a.batch * a.n_kv_head;
+  // One workgroup per compute unit; a tile of 64 keys takes 256 pairs 1.4 us there.
+  plan_splits(a, device_cus(), 1.4f,
+              a.window >= 0 ? std::min<int64_t>(a.t_max, a.window + QT) : a.t_max, p);
+  return p;
 }
 
 int launch_prefill_mfma(const AttnArgs &a) {
@@ -547,11 +593,19 @@ int launch_prefill_mfma(const AttnArgs &a) {
   P.cache_b = a.cache_batch_stride;
   P.scale_log2 = float(kLog2e / std::sqrt(double(D)));
   const int64_t n_qt = (a.t_new + P.QT - 1) / P.QT;
-  const int64_t blocks = n_qt * P.n_bh;
+  const SplitPlan plan = prefill_mfma_plan(a);
+  const SplitGeo geo = split_geo(a, plan);
+  const int64_t blocks = n_qt * P.n_bh * geo.n_split;
   if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
-  hipLaunchKernelGGL(prefill_mfma_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0,
-                     a.stream, P);
-  return launch_status("prefill_mfma");
+  if (geo.n_split == 1) {
+    hipLaunchKernelGGL(prefill_mfma_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, a.stream, P);
+    return launch_status("prefill_mfma");
+  }
+  hipLaunchKernelGGL(prefill_mfma_split_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, a.stream,
+                     P, geo);
+  const int st = launch_status("prefill_mfma");
+  if (st != MCAMD_OK) return st;
+  return launch_prefill_combine(a, geo, false);
 }
 
 }  // namespace mcamd

@@ -27,6 +27,11 @@
 //    the wave, so the weights are its B operand in place; the first takes dims 8c + i and
 //    8c + 4 + i, so that a lane reads its K row as 16-byte vectors.
 //
+// Measured against the VALU kernel this replaced (four lanes a row, an LDS float per FMA): four
+// 2048-token prompts of 12 heads of 64 in bf16 1858 -> 66 us (390 TFLOP/s of the attended pairs;
+// bound by the weights' exponentials and conversions on the VALU), in fp32 287 us (90 of the 144
+// TFLOP/s a large fp32 product reaches); two of 512 tokens in fp32 192 -> 30 us.
+//
 // Online softmax per pair in fp32 (exp2 domain): weights are made against the running maximum, and
 // the tile's own maximum is taken (and O rescaled) only when a lane's weights of the tile sum past
 // 2^15 or are not finite, or the pair has no maximum yet.
@@ -39,7 +44,7 @@
 // Not finite. The products multiply masked keys' values by a weight of zero, so an infinity or
 // NaN in V would reach pairs that may not see it, and an infinite value meets a zero lo term. A
 // pair whose result is not finite is therefore redone key by key, touching only the keys it sees.
-#include "kernels.h"
+#include "prefill_split.h"
 
 #include <cmath>
 #include <type_traits>
@@ -66,6 +71,7 @@ struct TiledParams {
   int T_new, H, H_kv, G, T_max, window, D, n_bh, n_qt;
   int64_t cache_b;
   float scale_log2;
+  SplitGeo split;
 };
 
 // Tile geometry of an instantiation (elements of E; DP is head_dim rounded up).
@@ -111,10 +117,11 @@ __device__ __forceinline__ bf16x4 lds_read_tr(const uint16_t *p) {
   return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16(lp));
 }
 
-// One pair redone by a wave, key by key over the keys it sees (lane l owns dims l, l + 64, ..):
-// for pairs whose result is not finite.
+// Dims [d0, d1) of one pair redone by a wave, key by key over the keys it sees (lane l owns dims
+// l, l + 64, ..): for pairs whose result is not finite.
 template <class E, int DP>
-__device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at, int p, int lane) {
+__device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at, int p, int lane,
+                             int d0, int d1) {
   constexpr int N = (DP + 63) / 64;
   const int D = P.D;
   const E *q = static_cast<const E *>(P.q) + at;
@@ -153,7 +160,7 @@ __device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at,
   const float inv = 1.f / l;
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    if (lane + 64 * i < D) out[lane + 64 * i] = from_f32<E>(o[i] * inv);
+    if (lane + 64 * i >= d0 && lane + 64 * i < d1) out[lane + 64 * i] = from_f32<E>(o[i] * inv);
 }
 
 // Four consecutive output dims.
@@ -176,7 +183,8 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   E *const sV = sK + KT * KSTR;
 
   const int bh = blockIdx.x % P.n_bh;
-  const int qt = P.n_qt - 1 - int(blockIdx.x / P.n_bh);
+  const int part = int(blockIdx.x / P.n_bh) % P.split.n_split;  // key range
+  const int qt = P.n_qt - 1 - int(blockIdx.x / P.n_bh) / P.split.n_split;
   const int b = bh / P.H_kv;
   const int kvh = bh - b * P.H_kv;
   const int row = P.rows ? P.rows[b] : b;
@@ -211,9 +219,26 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   const int64_t at = pair_at(pr);
   E *out = static_cast<E *>(P.out) + at;
   if (!row_ok) {
-    if (live && (KS == 1 || wave == 0))
+    if (live && part == 0 && (KS == 1 || wave == 0))
       for (int d = h; d < D; d += 2) out[d] = from_f32<E>(NAN);
     return;
+  }
+
+  const int p_abs = s0 + tq;
+  const int p_first = s0 + q0;
+  const int last = s0 + pair_pos(n - 1);  // the last key any pair of the workgroup sees
+  const int n_part = P.split.n_split;
+  int lo = P.window >= 0 ? max(0, p_first - P.window) : 0, hi = last;
+  int n_tiles = (hi - lo) / KT + 1;
+  bool whole = true;
+  if (n_part > 1) {  // this workgroup's range of the block's tiles
+    const int ranges = block_splits(P.split, s0, T_b, n_tiles);
+    if (part >= ranges) return;
+    whole = ranges == 1;
+    const int t0 = part * n_tiles / ranges, t1 = (part + 1) * n_tiles / ranges;
+    hi = min(hi, lo + t1 * KT - 1);
+    lo += t0 * KT;
+    n_tiles = t1 - t0;
   }
 
   // Q^T fragments, B[k = dim][n = pair]. bf16: dims 16 kd + 8h .. + 7 of step kd; fp32: dims
@@ -231,12 +256,6 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
       qf[i] = __builtin_bit_cast(QF, u);
     }
   }
-  const int p_abs = s0 + tq;
-  const int p_first = s0 + q0;
-  const int hi = s0 + pair_pos(n - 1);  // the last key any pair of the workgroup sees
-  const int lo = P.window >= 0 ? max(0, p_first - P.window) : 0;
-  const int n_tiles = (hi - lo) / KT + 1;
-
   const int64_t tok = int64_t(P.H_kv) * D;
   const E *kbase = static_cast<const E *>(P.k_cache) + int64_t(row) * P.cache_b + int64_t(kvh) * D;
   const E *vbase = static_cast<const E *>(P.v_cache) + int64_t(row) * P.cache_b + int64_t(kvh) * D;
@@ -314,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
       if constexpr (!kBf16) s[mk] = (sc[0] + sc[1]) + (sc[2] + sc[3]);
     }
     // Keys the pair may not see, in tiles that straddle the diagonal or the window's edge.
-    if (k0 + KW - 1 > p_first || (P.window >= 0 && k0 < hi - P.window)) {
+    if (k0 + KW - 1 > p_first || (P.window >= 0 && k0 < last - P.window)) {
 #pragma unroll
       for (int mk = 0; mk < MK; ++mk)
 #pragma unroll
@@ -393,6 +412,19 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
 
   l = sum_halves(l);
   if constexpr (KS == 1) {
+    if (!whole) {
+      if (!live) return;
+      const int64_t g = P.split.group(part, qt, bh, wave);
+#pragma unroll
+      for (int md = 0; md < MD; ++md)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (32 * md < D)
+            store4(P.split.o(g, md, j, lane), f32x4{o[md][4 * j], o[md][4 * j + 1],
+                                                    o[md][4 * j + 2], o[md][4 * j + 3]});
+      if (h == 0) *reinterpret_cast<float2 *>(P.split.ml(g, col)) = make_float2(m, l);
+      return;
+    }
     const float inv = 1.f / l;
     bool ok = true;
 #pragma unroll
@@ -417,7 +449,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
     }
     for (uint32_t left = bad; left != 0; left &= left - 1) {
       const int c = w0 + __builtin_ctz(left);
-      careful_pair<E, DP>(P, row, kvh, pair_at(c), s0 + pair_pos(c), lane);
+      careful_pair<E, DP>(P, row, kvh, pair_at(c), s0 + pair_pos(c), lane, 0, D);
     }
   } else {
     // Merge the four waves' (o, m, l) of the same 32 pairs; thread t then owns an eighth of the
@@ -449,7 +481,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
       // A wave that saw no key has l = 0; a NaN l (a NaN score) must stay.
       L += sm[kWaves * 32 + u * 32 + c] * (mu == -INFINITY ? 1.f : a[u]);
     }
-    const float inv = 1.f / L;
+    const float inv = whole ? 1.f / L : 1.f;
     constexpr int DT = DP / 8;
     f32x4 y[DT / 4];
     bool ok = true;
@@ -467,6 +499,16 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
       for (int e = 0; e < 4; ++e) ok = ok && (finite(y[i][e]) || d >= D);
     }
     const bool c_live = c < n;
+    if (!whole) {
+      if (!c_live) return;
+      const int64_t g = P.split.group(part, qt, bh, 0);
+      const int x = tid & 7;
+#pragma unroll
+      for (int i = 0; i < DT / 4; ++i)
+        if (32 * i < D) store4(P.split.o(g, i, x >> 1, 32 * (x & 1) + c), y[i]);
+      if (x == 0) *reinterpret_cast<float2 *>(P.split.ml(g, c)) = make_float2(M, L);
+      return;
+    }
     if (c_live && !ok) s_bad[c] = 1;
     __syncthreads();
     if (c_live && s_bad[c] == 0) {
@@ -479,48 +521,86 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
     }
     for (int x = wave; x < 32; x += kWaves) {
       if (s_bad[x] == 0) continue;
-      careful_pair<E, DP>(P, row, kvh, pair_at(x), s0 + pair_pos(x), lane);
+      careful_pair<E, DP>(P, row, kvh, pair_at(x), s0 + pair_pos(x), lane, 0, D);
     }
   }
 }
 
-template <class E, int DP, int KS>
-int run(TiledParams &P, int64_t pairs, hipStream_t stream) {
-  P.n_qt = int((pairs + Geo<E, DP, KS>::PAIRS - 1) / Geo<E, DP, KS>::PAIRS);
-  const int64_t blocks = int64_t(P.n_qt) * P.n_bh;
-  if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
-  hipLaunchKernelGGL((prefill_tiled_kernel<E, DP, KS>), dim3(unsigned(blocks)), dim3(kThreads), 0,
-                     stream, P);
-  return launch_status("prefill_tiled");
-}
-
-#ifndef MCAMD_TILED_KS4_BLOCKS
-#define MCAMD_TILED_KS4_BLOCKS 256
-#endif
-
-template <class E, int DP>
-int run_ks(TiledParams &P, int64_t pairs, hipStream_t stream) {
-  // Fewer workgroups of 128 pairs than fill the chip twice: 32 pairs and a quarter of the keys per
-  // wave instead. Head dims above 128 keep KS = 1 (a tile of four waves' keys outgrows the LDS).
-  if constexpr (DP <= 128) {
-    if ((pairs + 127) / 128 * P.n_bh < MCAMD_TILED_KS4_BLOCKS) return run<E, DP, 4>(P, pairs, stream);
-  }
-  return run<E, DP, 1>(P, pairs, stream);
-}
-
+// Merges the partials of key ranges, in the partials' own layout: a workgroup per 32 pairs and 32
+// dims, a wave per step j of them, eight ranges' loads in flight. Bound by the latency of those
+// loads at these sizes.
 template <class E>
-int dispatch(TiledParams &P, int64_t pairs, hipStream_t stream) {
-  if (P.D <= 32) return run_ks<E, 32>(P, pairs, stream);
-  if (P.D <= 64) return run_ks<E, 64>(P, pairs, stream);
-  if (P.D <= 96) return run_ks<E, 96>(P, pairs, stream);
-  if (P.D <= 128) return run_ks<E, 128>(P, pairs, stream);
-  if (P.D <= 192) return run_ks<E, 192>(P, pairs, stream);
-  return run_ks<E, 256>(P, pairs, stream);
+__global__ __launch_bounds__(256) void prefill_combine_kernel(TiledParams P, SplitGeo g,
+                                                              int careful) {
+  const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+  const int j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int md = blockIdx.x % g.md;
+  int at = blockIdx.x / g.md;
+  const int w = at % g.groups;
+  at /= g.groups;
+  const int bh = at % g.n_bh, qt = at / g.n_bh;
+  const int b = bh / P.H_kv, kvh = bh - b * P.H_kv;
+  const int d = 32 * md + 8 * j;  // this wave's dims d .. d + 7, lane half h d + 4h ..
+  const int s0 = P.seqlens[b];
+  if (d >= P.D || s0 < 0 || int64_t(s0) + P.T_new > P.T_max) return;  // NaN, written already
+  int lo, hi;
+  block_keys(g, s0, P.T_new, qt, lo, hi);
+  const int ranges = block_splits(g, s0, P.T_new, (hi - lo) / g.kt + 1);
+  if (ranges == 1) return;  // written by the block itself
+  const int64_t p0 = int64_t(qt) * g.pairs;
+  const int in_block = 32 * w + col;
+  const bool live = in_block < g.pairs && p0 + in_block < int64_t(P.T_new) * P.G;
+
+  constexpr int U = 8;
+  const int64_t group = g.group(0, qt, bh, w), step = g.group(1, qt, bh, w) - group;
+  const float *ml = g.ml(group, col);
+  const float *po = g.o(group, md, j, lane);
+  const int64_t ml_step = step * 64, o_step = step * g.md * 1024;
+  float M = -INFINITY, L = 0.f;
+  f32x4 y = {0.f, 0.f, 0.f, 0.f};
+  for (int r0 = 0; r0 < ranges; r0 += U) {
+    float2 x[U];
+    f32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int r = min(r0 + u, ranges - 1);
+      x[u] = *reinterpret_cast<const float2 *>(ml + r * ml_step);
+      v[u] = *reinterpret_cast<const f32x4 *>(po + r * o_step);
+    }
+    float m_new = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u) m_new = fmaxf(m_new, x[u].x);
+    const float keep = M == -INFINITY ? 0.f : fast_exp2(M - m_new);
+    L *= M == -INFINITY ? 1.f : keep;  // 0 then, or a NaN that must stay
+    y *= keep;
+    M = m_new;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (r0 + u >= ranges) break;
+      const float a = x[u].x == -INFINITY ? 0.f : fast_exp2(x[u].x - M);
+      L += x[u].y * (x[u].x == -INFINITY ? 1.f : a);
+      y += a * v[u];
+    }
+  }
+  y *= 1.f / L;
+  const bool ok = finite(y[0]) && finite(y[1]) && finite(y[2]) && finite(y[3]);
+  const int pos = live ? int((p0 + in_block) / P.G) : 0;
+  const int64_t row = (int64_t(b) * P.T_new + pos) * P.H + int64_t(kvh) * P.G +
+                      (live ? int(p0 + in_block - int64_t(pos) * P.G) : 0);
+  const uint64_t bad64 =
+      careful ? __builtin_amdgcn_ballot_w64(live && !ok && d + 4 * h < P.D) : 0;
+  const uint32_t bad = uint32_t(bad64) | uint32_t(bad64 >> 32);
+  if (live && !((bad >> col) & 1u) && d + 4 * h < P.D)
+    store4(static_cast<E *>(P.out) + row * P.D + d + 4 * h, y);
+  for (uint32_t left = bad; left != 0; left &= left - 1) {
+    const int c = __builtin_ctz(left);
+    const int rlo = __shfl(int(uint64_t(row)), c, 64), rhi = __shfl(int(uint64_t(row) >> 32), c, 64);
+    const int64_t r = int64_t((uint64_t(uint32_t(rhi)) << 32) | uint32_t(rlo));
+    careful_pair<E, 256>(P, b, kvh, r * P.D, s0 + __shfl(pos, c, 64), lane, d, min(d + 8, P.D));
+  }
 }
 
-}  // namespace
-
-int launch_prefill_tiled(const AttnArgs &a) {
+TiledParams tiled_params(const AttnArgs &a) {
   TiledParams P;
   P.q = a.q;
   P.k_cache = a.k_cache;
@@ -533,16 +613,106 @@ int launch_prefill_tiled(const AttnArgs &a) {
   P.H = int(a.n_head);
   P.H_kv = int(a.n_kv_head);
   P.G = int(a.n_head / a.n_kv_head);
-  if (P.G > 64) return fail(MCAMD_EUNSUPPORTED, "prefill: more than 64 query heads per KV head");
   P.T_max = int(a.t_max);
   P.window = int(a.window < 0 ? -1 : a.window);
   P.D = int(a.head_dim);
   P.n_bh = int(a.batch * a.n_kv_head);
+  P.n_qt = 0;
   P.cache_b = a.cache_batch_stride;
   P.scale_log2 = float(kLog2e / std::sqrt(double(a.head_dim)));
-  const int64_t pairs = a.t_new * P.G;
-  if (a.dtype == MCAMD_BF16) return dispatch<bf16>(P, pairs, a.stream);
-  return dispatch<float>(P, pairs, a.stream);
+  P.split = SplitGeo{};
+  P.split.n_split = 1;
+  return P;
+}
+
+
+// What a call runs: the waves over pairs (KS = 1) or keys (KS = 4), and the key ranges.
+struct TiledPlan {
+  int ks;
+  SplitPlan split;
+};
+TiledPlan tiled_plan(const AttnArgs &a) {
+  const int64_t G = a.n_head / a.n_kv_head;
+  const int64_t n_bh = a.batch * a.n_kv_head;
+  const bool bf = a.dtype == MCAMD_BF16;
+  TiledPlan t;
+  SplitPlan &p = t.split;
+  // Fewer workgroups of 128 pairs than compute units: 32 pairs and a quarter of the keys per wave
+  // instead (12 heads of 64: 2 x 512 tokens fp32 33 against 50 us, bf16 15.0 against 18.6; 8 x 512,
+  // 384 workgroups: 78 against 67 and 31.6 against 21.8). Head dims above 128 keep KS = 1 (a tile of four waves' keys outgrows the LDS).
+  t.ks = a.head_dim <= 128 && (a.t_new * G + 127) / 128 * n_bh < 256 ? 4 : 1;
+  p.pairs = 128 / t.ks;
+  p.kt = t.ks == 4 ? 128 : bf && a.head_dim <= 128 ? 64 : 32;
+  p.blocks = (a.t_new * G + p.pairs - 1) / p.pairs * n_bh;
+  // Measured time of a tile on a compute unit of its own, per head dim. The chip counts as full at
+  // one workgroup per compute unit: cutting 192 blocks in two gains on long prefixes (512 tokens of
+  // 12 heads of 64 after 4096 keys, bf16: 52 against 63 us) what it loses on short ones (from
+  // empty: 17 against 11.6).
+  const float tile_us = float(a.head_dim) * (t.ks == 4 ? (bf ? 0.027f : 0.085f)
+                                                       : (bf ? 0.012f : 0.035f));
+  plan_splits(a, device_cus(), tile_us,
+              a.window >= 0 ? std::min<int64_t>(a.t_max, a.window + 1 + (p.pairs + G - 1) / G)
+                            : a.t_max, p);
+  return t;
+}
+
+template <class E, int DP, int KS>
+int run(TiledParams &P, const AttnArgs &a, const TiledPlan &plan) {
+  using G_ = Geo<E, DP, KS>;
+  if (plan.split.pairs != G_::PAIRS || plan.split.kt != G_::KT)
+    return fail(MCAMD_EINVAL, "prefill: plan and kernel disagree");
+  P.split = split_geo(a, plan.split);
+  P.n_qt = P.split.n_qt;
+  const int64_t blocks = plan.split.blocks * P.split.n_split;
+  if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
+  hipLaunchKernelGGL((prefill_tiled_kernel<E, DP, KS>), dim3(unsigned(blocks)), dim3(kThreads), 0,
+                     a.stream, P);
+  const int st = launch_status("prefill_tiled");
+  if (st != MCAMD_OK || P.split.n_split == 1) return st;
+  return launch_prefill_combine(a, P.split, true);
+}
+
+template <class E, int DP>
+int run_ks(TiledParams &P, const AttnArgs &a, const TiledPlan &plan) {
+  if constexpr (DP <= 128) {
+    if (plan.ks == 4) return run<E, DP, 4>(P, a, plan);
+  }
+  return run<E, DP, 1>(P, a, plan);
+}
+
+template <class E>
+int dispatch(TiledParams &P, const AttnArgs &a, const TiledPlan &plan) {
+  if (P.D <= 32) return run_ks<E, 32>(P, a, plan);
+  if (P.D <= 64) return run_ks<E, 64>(P, a, plan);
+  if (P.D <= 96) return run_ks<E, 96>(P, a, plan);
+  if (P.D <= 128) return run_ks<E, 128>(P, a, plan);
+  if (P.D <= 192) return run_ks<E, 192>(P, a, plan);
+  return run_ks<E, 256>(P, a, plan);
+}
+
+}  // namespace
+
+int launch_prefill_combine(const AttnArgs &a, const SplitGeo &g, bool careful) {
+  const TiledParams P = tiled_params(a);
+  const int64_t blocks = int64_t(g.n_qt) * g.n_bh * g.groups * g.md;
+  if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
+  const dim3 grid{unsigned(blocks)}, threads{256};
+  if (a.dtype == MCAMD_BF16)
+    hipLaunchKernelGGL(prefill_combine_kernel<bf16>, grid, threads, 0, a.stream, P, g, int(careful));
+  else
+    hipLaunchKernelGGL(prefill_combine_kernel<float>, grid, threads, 0, a.stream, P, g, int(careful));
+  return launch_status("prefill_combine");
+}
+
+SplitPlan prefill_tiled_splits(const AttnArgs &a) { return tiled_plan(a).split; }
+
+int launch_prefill_tiled(const AttnArgs &a) {
+  TiledParams P = tiled_params(a);
+  if (P.G > 64) return fail(MCAMD_EUNSUPPORTED, "prefill: more than 64 query heads per KV head");
+  const TiledPlan plan = tiled_plan(a);
+  if (plan.split.blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
+  if (a.dtype == MCAMD_BF16) return dispatch<bf16>(P, a, plan);
+  return dispatch<float>(P, a, plan);
 }
 
 }  // namespace mcamd

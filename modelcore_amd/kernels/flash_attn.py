@@ -202,8 +202,12 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, cache_seqlens=N
     out = torch.empty((B, T_new, H, D), dtype=dt, device=q.device)
     lib = _ext.lib()
     w = _window(window_size)
-    ws_bytes = lib.mcamd_attn_workspace_bytes(B, T_new, H, H_kv, D, T_max, w)
-    ws = _ext.workspace(q.device, ws_bytes)
+    if T_new == 1:
+        ws = _ext.workspace(q.device, lib.mcamd_attn_workspace_bytes(B, 1, H, H_kv, D, T_max, w))
+    else:
+        # Scratch of the call's own: prefills on several streams share nothing.
+        ws_bytes = lib.mcamd_attn_scratch_bytes(B, T_new, H, H_kv, D, T_max, w, code)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     args = (q.data_ptr(), k.data_ptr() if k is not None else None,
             v.data_ptr() if v is not None else None, k_cache.data_ptr(), v_cache.data_ptr(),
             seqlens.data_ptr(), out.data_ptr(), B, T_new, H, H_kv, D, T_max, k_cache.stride(0), w,

@@ -1,5 +1,5 @@
 """The matrix-core chunked prefill for fp32 caches and head dims other than 128
-(prefill_tiled.hip), at the edges of its tiles: 32 and 128 pairs per workgroup, 32, 64 and 128
+(prefill_tiled.hip), and the key ranges of calls with few query blocks (prefill_split.h), at the edges of its tiles: 32 and 128 pairs per workgroup, 32, 64 and 128
 keys per tile, every head-dim instantiation with and without padded dims.
 
 Tolerance: bf16 rounds the output once (at most 2^-8 of it: 8 bits) and holds the weights to 2^-17, so the sums
@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from _util import ATOL, make_case, to_np
+from modelcore_amd import _ext
 from modelcore_amd.kernels.flash_attn import flash_attn
 from oracle import kv_oracle as ko
 
@@ -95,3 +96,65 @@ def test_infinities_and_nan_reach_only_the_pairs_that_see_them(dtype, heads):
     _close(out[1, 20:, :, 10:], ref[1, 20:, :, 10:], dtype)
     _close(out[2, :35], ref[2, :35], dtype)
     assert torch.equal(out[3], plain[3])
+
+
+SPLIT_CASES = [
+    # seqlens, T_new, H, H_kv, D, T_max, window
+    ([8000], 100, 32, 8, 128, 8200, -1),          # two blocks of queries, many ranges
+    ([3000, 17], 40, 12, 12, 64, 3100, -1),       # a long row beside one that is not cut
+    ([0, 900], 300, 2, 2, 128, 1300, -1),         # blocks of one to many tiles, from an empty cache
+    ([2000, 1500], 30, 4, 1, 256, 2100, -1),
+    ([2500], 50, 10, 2, 96, 2600, 1500),          # a window that starts inside the first range
+    ([1000, 5], 70, 6, 2, 128, 4000, 700),        # a cache far longer than the rows
+    ([511, 512, 513], 2, 4, 4, 72, 516, -1),      # ranges of about the least length
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("seqlens,T_new,H,H_kv,D,T_max,window", SPLIT_CASES)
+def test_key_ranges_match_the_oracle(dtype, seqlens, T_new, H, H_kv, D, T_max, window):
+    """bf16 at head_dim 128 keeps that kernel's tolerance (its weights are bf16)."""
+    print("case: ranges", dtype, seqlens, T_new, H, H_kv, D, T_max, window, flush=True)
+    scratch = _ext.lib().mcamd_attn_scratch_bytes(len(seqlens), T_new, H, H_kv, D, T_max, window,
+                                                  _ext.dtype_code(dtype))
+    assert scratch >= 2 * len(seqlens) * T_new * H * (D + 2) * 4  # at least two ranges
+    c = make_case(seqlens, T_new, H, H_kv, D, T_max, dtype, seed=43)
+    out, ref = _run(c, window), _oracle(c, window)
+    if dtype == torch.bfloat16 and D == 128:
+        assert np.abs(to_np(out) - ref).max() <= ATOL[dtype]
+    else:
+        _close(out, ref, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [64, 128])
+def test_key_ranges_with_rows_outside_the_cache_and_non_finite_values(dtype, D):
+    print("case: ranges, bad rows", dtype, D, flush=True)
+    seqlens, T_new, H, H_kv, T_max = [1990, 1200, -1], 33, 4, 2, 2000
+    c = make_case([1900, 1200, 0], T_new, H, H_kv, D, T_max, dtype, seed=44)
+    good = _run(c, -1)
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    c["v_cache"][1, 100, 0, 3] = float("inf")
+    out = _run(c, -1)
+    assert torch.isnan(out[0]).all() and torch.isnan(out[2]).all()
+    assert torch.equal(out[1, :, 2:], good[1, :, 2:])  # the other KV head's queries
+    if dtype == torch.float32 or D != 128:
+        assert torch.isposinf(out[1, :, :2, 3]).all()
+        assert torch.isfinite(out[1, :, :2, :3]).all() and torch.isfinite(out[1, :, :2, 4:]).all()
+
+
+def test_without_scratch_the_keys_stay_whole():
+    """The C entry without a workspace gives the same call within its rounding, and the same bits
+    whatever stream it runs on."""
+    print("case: ranges, no scratch", flush=True)
+    c = make_case([2000, 31], 20, 8, 2, 64, 2100, torch.float32, seed=45)
+    out = _run(c, -1)
+    g = _gpu(c)
+    whole = torch.empty_like(g["q"])
+    st = _ext.lib().mcamd_flash_attn_with_kvcache(
+        g["q"].data_ptr(), g["k"].data_ptr(), g["v"].data_ptr(), g["k_cache"].data_ptr(),
+        g["v_cache"].data_ptr(), g["cache_seqlens"].data_ptr(), whole.data_ptr(), 2, 20, 8, 2, 64,
+        2100, g["k_cache"].stride(0), -1, 1, _ext.F32, None, 0, _ext.stream_handle(DEV))
+    _ext.check(st, "no scratch")
+    _close(whole, _oracle(c, -1), torch.float32)
+    _close(out, _oracle(c, -1), torch.float32)
