@@ -54,6 +54,7 @@
 //
 // The shared prompt prefix of a decode step runs inside the fused decode kernel (prefix_mfma.h),
 // built from the same fragments and layouts.
+#include "prefill_order.h"
 #include "prefill_split.h"
 
 #include <cmath>
@@ -81,7 +82,7 @@ struct MfmaParams {
   const int32_t *seqlens;
   const int32_t *rows, *cu;  // varlen prefill (optional): cache row and token range per sequence
   uint16_t *out;
-  int T_new, H, H_kv, G, QT, T_max, window, n_bh;
+  int T_new, H, H_kv, G, QT, T_max, window, n_bh, n_qt, descend;
   int64_t cache_b;
   float scale_log2;
 };
@@ -145,32 +146,55 @@ __device__ __forceinline__ float exp2_or_zero(float x) {
   return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x);
 }
 
-// SPLIT: a workgroup per key range of a block (prefill_split.h).
-template <bool SPLIT>
+// SPLIT: a workgroup per key range of a block (prefill_split.h). VARLEN: sequences of their own
+// lengths, packed along the token axis.
+template <bool SPLIT, bool VARLEN>
 __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const SplitGeo *S) {
   __shared__ __attribute__((aligned(1024))) uint16_t sK[4][TILE];
   __shared__ __attribute__((aligned(1024))) uint16_t sV[4][TILE];
 
-  const int bh = blockIdx.x % P.n_bh;
-  const int rest = blockIdx.x / P.n_bh;
-  const int part = SPLIT ? rest % S->n_split : 0;  // key range
-  const int qt = SPLIT ? rest / S->n_split : rest;
-  const int b = bh / P.H_kv;  // sequence (a cache row, or one prompt of a varlen batch)
-  const int kvh = bh - b * P.H_kv;
-  const int q0 = qt * P.QT;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
+  int bh = blockIdx.x % P.n_bh;
+  const int rest = blockIdx.x / P.n_bh;
+  const int part = SPLIT ? rest % S->n_split : 0;  // key range
+  int qt = SPLIT ? rest / S->n_split : rest;
+  // The longest blocks, a prompt's last, first (two prompts of 4096 tokens, 12 / 4 heads: 147 us in
+  // the other order, 118 so). With a window most are alike, and ascending they share its keys in
+  // L2 (eight of 2048 tokens, window 1024: 113 us, 115 descending); blocks that all start at once
+  // gain nothing either (one of 2048 tokens, 256 blocks: 58.5 us, 60.3 descending).
+  if (P.descend) qt = P.n_qt - 1 - qt;
+  int b = bh / P.H_kv;  // sequence (a cache row, or one prompt of a varlen batch)
+  int kvh = bh - b * P.H_kv;
+  // Varlen: sequence b's queries are tokens [cu[b], cu[b + 1]) of q/out, its keys cache row
+  // rows[b]; a query tile past the sequence's end has nothing to do (a whole workgroup).
+  int row = b, T_b = P.T_new, s0;
+  int64_t tok0 = int64_t(b) * P.T_new;
+  if constexpr (VARLEN) {
+    const int n_seqs = P.n_bh / P.H_kv;
+    if (n_seqs <= kOrderedSeqs) {
+      VarlenBlock v;
+      if (!find_varlen_block(P.cu, P.rows, P.seqlens, n_seqs, P.n_qt, P.QT * P.G, P.G,
+                             int(blockIdx.x) / P.H_kv, lane, v))
+        return;
+      kvh = int(blockIdx.x) % P.H_kv;
+      bh = v.b * P.H_kv + kvh;
+      b = v.b, qt = v.qt, row = v.row, tok0 = v.tok0, T_b = v.T_b, s0 = v.s0;
+    } else {
+      row = P.rows ? P.rows[b] : b;
+      tok0 = P.cu[b];
+      T_b = P.cu[b + 1] - P.cu[b];
+      s0 = P.seqlens[row];
+    }
+  } else {
+    s0 = P.seqlens[row];
+  }
+  const int q0 = qt * P.QT;
   const int wave = tid >> 6;
   const int h = lane >> 5;    // lane half
   const int col = lane & 31;  // this lane's pair within the wave's 32
 
-  // Varlen: sequence b's queries are tokens [cu[b], cu[b + 1]) of q/out, its keys cache row
-  // rows[b]; a query tile past the sequence's end has nothing to do (a whole workgroup).
-  const int row = P.rows ? P.rows[b] : b;
-  const int64_t tok0 = P.cu ? int64_t(P.cu[b]) : int64_t(b) * P.T_new;
-  const int T_b = P.cu ? P.cu[b + 1] - P.cu[b] : P.T_new;
   if (q0 >= T_b) return;
-  const int s0 = P.seqlens[row];
   const int q_end = min(q0 + P.QT, T_b);  // positions [q0, q_end) of the chunk
   const bool row_ok = s0 >= 0 && int64_t(s0) + T_b <= P.T_max;
 
@@ -541,10 +565,13 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
 }
 
 __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P) {
-  prefill_mfma_body<false>(P, nullptr);
+  prefill_mfma_body<false, false>(P, nullptr);
+}
+__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_varlen_kernel(MfmaParams P) {
+  prefill_mfma_body<false, true>(P, nullptr);
 }
 __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_split_kernel(MfmaParams P, SplitGeo S) {
-  prefill_mfma_body<true>(P, &S);
+  prefill_mfma_body<true, false>(P, &S);
 }
 
 }  // namespace
@@ -590,13 +617,20 @@ int launch_prefill_mfma(const AttnArgs &a) {
   P.T_max = int(a.t_max);
   P.window = int(a.window < 0 ? -1 : a.window);
   P.n_bh = int(a.batch * a.n_kv_head);
+  P.n_qt = int((a.t_new + P.QT - 1) / P.QT);
   P.cache_b = a.cache_batch_stride;
   P.scale_log2 = float(kLog2e / std::sqrt(double(D)));
-  const int64_t n_qt = (a.t_new + P.QT - 1) / P.QT;
   const SplitPlan plan = prefill_mfma_plan(a);
   const SplitGeo geo = split_geo(a, plan);
-  const int64_t blocks = n_qt * P.n_bh * geo.n_split;
+  P.descend = P.window < 0 && int64_t(P.n_qt) * P.n_bh > device_cus();
+  const int64_t blocks = int64_t(P.n_qt) * P.n_bh * geo.n_split;
   if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "prefill: grid too large");
+  if (a.cu) {
+    hipLaunchKernelGGL(prefill_mfma_varlen_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0,
+                       a.stream, P);
+    return launch_status("prefill_mfma");
+  }
+  if (a.rows) return fail(MCAMD_EINVAL, "prefill: rows come with cu_seqlens");
   if (geo.n_split == 1) {
     hipLaunchKernelGGL(prefill_mfma_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, a.stream, P);
     return launch_status("prefill_mfma");

@@ -44,6 +44,7 @@
 // Not finite. The products multiply masked keys' values by a weight of zero, so an infinity or
 // NaN in V would reach pairs that may not see it, and an infinite value meets a zero lo term. A
 // pair whose result is not finite is therefore redone key by key, touching only the keys it sees.
+#include "prefill_order.h"
 #include "prefill_split.h"
 
 #include <cmath>
@@ -182,14 +183,29 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   E *const sK = reinterpret_cast<E *>(s_raw);
   E *const sV = sK + KT * KSTR;
 
-  const int bh = blockIdx.x % P.n_bh;
+  int bh = blockIdx.x % P.n_bh;
   const int part = int(blockIdx.x / P.n_bh) % P.split.n_split;  // key range
-  const int qt = P.n_qt - 1 - int(blockIdx.x / P.n_bh) / P.split.n_split;
-  const int b = bh / P.H_kv;
-  const int kvh = bh - b * P.H_kv;
-  const int row = P.rows ? P.rows[b] : b;
-  const int64_t tok0 = P.cu ? int64_t(P.cu[b]) : int64_t(b) * P.T_new;
-  const int T_b = P.cu ? P.cu[b + 1] - P.cu[b] : P.T_new;
+  int qt = P.n_qt - 1 - int(blockIdx.x / P.n_bh) / P.split.n_split;
+  int b = bh / P.H_kv;
+  int kvh = bh - b * P.H_kv;
+  int row = b, T_b = P.T_new, s0;
+  int64_t tok0 = int64_t(b) * P.T_new;
+  if (P.cu && P.n_bh <= kOrderedSeqs * P.H_kv) {
+    VarlenBlock v;
+    if (!find_varlen_block(P.cu, P.rows, P.seqlens, P.n_bh / P.H_kv, P.n_qt, G_::PAIRS, P.G,
+                           int(blockIdx.x) / P.H_kv, threadIdx.x & 63, v))
+      return;
+    kvh = int(blockIdx.x) % P.H_kv;
+    bh = v.b * P.H_kv + kvh;
+    b = v.b, qt = v.qt, row = v.row, tok0 = v.tok0, T_b = v.T_b, s0 = v.s0;
+  } else {
+    if (P.cu) {
+      row = P.rows ? P.rows[b] : b;
+      tok0 = P.cu[b];
+      T_b = P.cu[b + 1] - P.cu[b];
+    }
+    s0 = P.seqlens[row];
+  }
   // This workgroup's pairs: n of them from pair p0 on, which is head r0 of position q0.
   const int64_t n_pairs = int64_t(T_b) * P.G;
   const int64_t p0 = int64_t(qt) * G_::PAIRS;
@@ -204,7 +220,6 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   const int col = lane & 31;  // this lane's pair within the wave's 32
   const int D = P.D;
 
-  const int s0 = P.seqlens[row];
   const bool row_ok = s0 >= 0 && int64_t(s0) + T_b <= P.T_max;
   const int w0 = KS == 1 ? 32 * wave : 0;  // the wave's first pair
   const bool live = w0 + col < n;

@@ -98,6 +98,32 @@ def test_varlen_matches_the_oracle_per_sequence(dtype, H, H_kv, D, T_max, B_cach
     assert torch.equal(after, moved), "advance moves exactly the listed rows by their lengths"
 
 
+ORDER_CASES = [
+    # lengths of the sequences: launch order by block number across sequences, up to 64 of them
+    [500, 3, 260, 0, 129, 1, 400, 64],            # ragged, one empty
+    [(37 * i) % 90 for i in range(64)],           # exactly 64 sequences
+    [(37 * i) % 50 + 1 for i in range(65)],       # more: an id per (sequence, block)
+    [700],
+]
+
+
+@pytest.mark.parametrize("lengths", ORDER_CASES, ids=["ragged", "64", "65", "one"])
+@pytest.mark.parametrize("dtype,D,window", [(torch.bfloat16, 128, -1), (torch.bfloat16, 128, 60),
+                                            (torch.bfloat16, 64, -1), (torch.float32, 64, 45)])
+def test_every_block_of_every_sequence_is_launched(dtype, D, window, lengths):
+    _note("varlen order", dtype, D, window, lengths)
+    n = len(lengths)
+    rows = [(i * 7 + 3) % n for i in range(n)] if n % 7 else list(range(n))
+    bases = [(11 * i) % 40 for i in range(n)]
+    c = _case(dtype, 6, 2, D, max(lengths) + 40, n, lengths, seed=64)
+    out, _, _, _ = _run(c, rows, bases, lengths, window)
+    keep = [i for i in range(n) if lengths[i] > 0]  # the oracle takes no empty sequence
+    want, _, _ = _oracle(c, [rows[i] for i in keep], [bases[i] for i in keep],
+                         [lengths[i] for i in keep], window)
+    err = max_abs(to_np(out), want)
+    assert err <= ATOL[dtype], f"max-abs {err}"
+
+
 def test_varlen_without_rows_uses_rows_in_order_and_leaves_positions():
     c = _case(torch.bfloat16, 16, 4, 128, 160, 3, [60, 1, 99], seed=62)
     out, g, after, before = _run(c, [0, 1, 2], [0, 50, 7], [60, 1, 99], -1)
