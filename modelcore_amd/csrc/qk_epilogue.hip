@@ -179,6 +179,172 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void qk_epilogue_kernel(
   }
 }
 
+// The same step in 16-byte pieces, where every row is made of them (a half head of whole pieces,
+// 16-byte aligned rows and tables): LPI lanes per head, lane L holding dims VEC L .. + VEC - 1 of the
+// first half and their rotation partners in the second, so 64 / LPI heads per wave.
+// Bound by memory: 8 x 512 tokens of 32 + 2 x 8 heads of 128 in bf16 move 101 MB in 20.6 us (4.9
+// TB/s; a large copy 5.2), against 75.3 for the wave per head above, whose 2-byte accesses and
+// one-value-at-a-time rounding bound it; 64 single tokens of it 3.51 against 3.75 us.
+//
+// The sum of squares is added in the order of the wave per head, so that both give the same bits:
+// there lane j < 64 adds dims j, j + D/2 (and j + 64, j + 64 + D/2 after them), and the lanes are
+// added in steps of 32, 16, .., 1. Here steps of VEC and more go over the lanes, the rest within one.
+template <class E>
+struct Pieces;
+template <>
+struct Pieces<bf16> {
+  static constexpr int N = 8;
+  typedef float F __attribute__((ext_vector_type(8)));
+  typedef __bf16 H __attribute__((ext_vector_type(8)));
+  static __device__ __forceinline__ F load(const bf16 *p) {
+    return __builtin_convertvector(__builtin_bit_cast(H, *reinterpret_cast<const uint4 *>(p)), F);
+  }
+  static __device__ __forceinline__ void store(bf16 *p, const F &x) {
+    *reinterpret_cast<uint4 *>(p) = __builtin_bit_cast(uint4, __builtin_convertvector(x, H));
+  }
+  static __device__ __forceinline__ F rnd(const F &x) {
+    return __builtin_convertvector(__builtin_convertvector(x, H), F);
+  }
+};
+template <>
+struct Pieces<float> {
+  static constexpr int N = 4;
+  typedef float F __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ F load(const float *p) {
+    return *reinterpret_cast<const F *>(p);
+  }
+  static __device__ __forceinline__ void store(float *p, const F &x) {
+    *reinterpret_cast<F *>(p) = x;
+  }
+  static __device__ __forceinline__ F rnd(const F &x) { return x; }
+};
+
+template <class T, int LPI>
+__global__ __launch_bounds__(64 * kWavesPerBlock) void qk_epilogue_pieces_kernel(
+    const int32_t *a_seqlens, const void *a_q, int64_t a_q_tok, int a_n_rows, int a_n_items,
+    int a_t_new, int a_D, int a_H, EpiParams P) {
+#pragma clang fp contract(off)
+  typedef Pieces<T> V;
+  typedef typename V::F F;
+  constexpr int N = V::N;
+  const int row = int((blockIdx.x * (64 * kWavesPerBlock) + threadIdx.x) / LPI);
+  const int L = threadIdx.x % LPI;
+  const bool here = row < a_n_rows;
+  const int tok = here ? row / a_n_items : 0;
+  const int item = here ? row - tok * a_n_items : 0;
+  const int b = tok / a_t_new;
+  const int64_t pos = int64_t(a_seqlens[b]) + (tok - b * a_t_new);
+  const int half = a_D >> 1;
+  const int j = N * L;
+  const bool mine = here && j < half;  // this lane holds dims of the head
+  const bool in_table = pos >= 0 && pos < P.n_pos;
+  const bool in_cache = pos >= 0 && pos < P.t_max;
+  const bool is_q = item < a_H, is_v = item >= a_H + P.H_kv;
+
+  const T *src;
+  T *dst;
+  if (is_q) {
+    src = static_cast<const T *>(a_q) + int64_t(tok) * a_q_tok + int64_t(item) * a_D;
+    dst = static_cast<T *>(P.q_out) + (int64_t(tok) * a_H + item) * a_D;
+  } else {
+    const int hk = item - a_H - (is_v ? P.H_kv : 0);
+    src = (is_v ? static_cast<const T *>(P.v) + int64_t(tok) * P.v_tok
+                : static_cast<const T *>(P.k) + int64_t(tok) * P.k_tok) + int64_t(hk) * a_D;
+    dst = static_cast<T *>(is_v ? P.v_cache : P.k_cache) + int64_t(b) * P.cache_b +
+          (pos * P.H_kv + hk) * a_D;
+  }
+  src += j;
+  dst += j;
+  if (is_v && mine && in_cache) {  // a plain copy
+    const uint4 x = *reinterpret_cast<const uint4 *>(src);
+    const uint4 y = *reinterpret_cast<const uint4 *>(src + half);
+    *reinterpret_cast<uint4 *>(dst) = x;
+    *reinterpret_cast<uint4 *>(dst + half) = y;
+  }
+  const bool rotates = mine && !is_v && in_table && (is_q || in_cache);
+  F y1, y2, ss;
+#pragma unroll
+  for (int e = 0; e < N; ++e) y1[e] = y2[e] = ss[e] = 0.f;
+  if (rotates) {
+    const F x1 = V::load(src), x2 = V::load(src + half);
+    const F c = V::load(static_cast<const T *>(P.cos) + pos * half + j);
+    const F s = V::load(static_cast<const T *>(P.sin) + pos * half + j);
+    y1 = V::rnd(V::rnd(x1 * c) + V::rnd(x2 * s));
+    y2 = V::rnd(V::rnd(x1 * -s) + V::rnd(x2 * c));
+  }
+#pragma unroll
+  for (int e = 0; e < N; ++e) ss[e] = fmaf(y2[e], y2[e], fmaf(y1[e], y1[e], 0.f));
+  if constexpr (LPI * N > 64) {  // dims j + 64 after dims j, in the lanes that hold them
+    constexpr int kOff = 64 / N;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const float first = __shfl_xor(ss[e], kOff, 64);
+      const float both = fmaf(y2[e], y2[e], fmaf(y1[e], y1[e], first));
+      const float back = __shfl_xor(both, kOff, 64);
+      ss[e] = (L & kOff) ? both : back;
+    }
+  }
+#pragma unroll
+  for (int o = (LPI * N > 64 ? 64 : LPI * N) / 2; o >= N; o >>= 1)
+#pragma unroll
+    for (int e = 0; e < N; ++e) ss[e] += __shfl_xor(ss[e], o / N, 64);
+#pragma unroll
+  for (int o = N / 2; o > 0; o >>= 1)
+#pragma unroll
+    for (int e = 0; e < o; ++e) ss[e] += ss[e + o];
+  if (!mine || is_v) return;
+  if (!in_table) {
+    if (is_q) {
+      F nan;
+#pragma unroll
+      for (int e = 0; e < N; ++e) nan[e] = NAN;
+      V::store(dst, nan);
+      V::store(dst + half, nan);
+    }
+    return;
+  }
+  if (!rotates) return;
+  const float inv = __fdiv_rn(1.f, __fsqrt_rn(__fdiv_rn(ss[0], float(a_D)) + P.eps));
+  V::store(dst, V::rnd(y1 * inv) * P.scale);
+  V::store(dst + half, V::rnd(y2 * inv) * P.scale);
+}
+
+template <class T>
+bool launch_pieces(const EpiParams &P, hipStream_t stream) {
+  constexpr int N = Pieces<T>::N;
+  const int64_t size = sizeof(T);
+  const int half = P.D / 2;
+  const bool with_kv = P.k != nullptr;
+  const int64_t rows = P.n_tokens * P.n_items;
+  auto pieces = [&](const void *p, int64_t stride) {
+    return aligned(p, 16) && stride * size % 16 == 0;
+  };
+  if (P.D % 2 != 0 || half % N != 0 || rows * 64 > 0x7fffffff || !pieces(P.q, P.q_tok) ||
+      !pieces(P.q_out, P.D) || !pieces(P.cos, half) || !pieces(P.sin, half) ||
+      (with_kv && (!pieces(P.k, P.k_tok) || !pieces(P.v, P.v_tok) ||
+                   !pieces(P.k_cache, P.cache_b) || !pieces(P.v_cache, P.cache_b))))
+    return false;
+  int lpi = 1;
+  while (lpi * N < half) lpi *= 2;
+  const int64_t threads = rows * lpi;
+  const dim3 grid{unsigned((threads + 64 * kWavesPerBlock - 1) / (64 * kWavesPerBlock))};
+  const dim3 block{64 * kWavesPerBlock};
+#define MCAMD_PIECES(LPI)                                                                          \
+  hipLaunchKernelGGL((qk_epilogue_pieces_kernel<T, LPI>), grid, block, 0, stream, P.seqlens, P.q,  \
+                     P.q_tok, int(rows), P.n_items, P.t_new, P.D, P.H, P)
+  switch (lpi) {
+    case 1: MCAMD_PIECES(1); break;
+    case 2: MCAMD_PIECES(2); break;
+    case 4: MCAMD_PIECES(4); break;
+    case 8: MCAMD_PIECES(8); break;
+    case 16: MCAMD_PIECES(16); break;
+    default:  // 32: fp32 past head_dim 128
+      if constexpr (N == 4) MCAMD_PIECES(32);
+  }
+#undef MCAMD_PIECES
+  return true;
+}
+
 }  // namespace
 }  // namespace mcamd
 
@@ -243,6 +409,10 @@ extern "C" int mcamd_qk_rope_norm_append(const void *q, int64_t q_token_stride, 
   P.scale = scale;
   if (t_new > 0x7fffffff || n_head + 2 * n_kv_head > 0x7fffffff)
     return fail(MCAMD_EUNSUPPORTED, "qk_rope_norm_append: sizes too large");
+  // Rows of whole 16-byte pieces; others, and calls past 32-bit thread numbers, take a wave per head.
+  if (dtype == MCAMD_BF16 ? launch_pieces<bf16>(P, as_stream(stream))
+                          : launch_pieces<float>(P, as_stream(stream)))
+    return launch_status("qk_rope_norm_append");
   const int64_t waves = P.n_tokens * P.n_items;
   const int64_t blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
   if (blocks > 0x7fffffff) return fail(MCAMD_EUNSUPPORTED, "qk_rope_norm_append: grid too large");

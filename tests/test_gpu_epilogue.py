@@ -94,6 +94,30 @@ def test_strided_views_of_a_fused_projection_are_read_in_place(T):
     assert torch.equal(a, b) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [8, 16, 64, 80, 96, 128, 144, 192, 256])
+def test_both_kernels_give_the_same_bits(dtype, D):
+    """Rows of whole 16-byte pieces take a kernel of their own; the same values one element off
+    take the wave per head. Same bits, also past the table and the cache."""
+    _note("epilogue pieces", dtype, D)
+    B, T, H, H_kv, T_max, n_pos = 3, 9, 6, 2, 30, 28
+    c = _case(7, B, T, H, H_kv, D, T_max, n_pos, dtype, [0, 15, 24])
+
+    def off(t):  # the same values at an address past a 16-byte boundary
+        return torch.cat([t.new_zeros(1), t.reshape(-1)]).to(DEV)[1:].view(t.shape)
+
+    outs = []
+    for put in (lambda t: t.to(DEV), off):
+        kc, vc = c["kc"].to(DEV), c["vc"].to(DEV)
+        q = rope_norm_scale_append(put(c["q"]), c["cos"].to(DEV), c["sin"].to(DEV),
+                                   c["seqlens"].to(DEV), put(c["k"]), put(c["v"]), kc, vc)
+        outs.append((q, kc, vc))
+    for a, b in zip(*outs):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+        assert torch.equal(a.nan_to_num(), b.nan_to_num())
+    assert torch.isnan(outs[0][0][2, 4:]).all() and not torch.isnan(outs[0][0][2, :4]).any()
+
+
 def test_queries_only_for_kv_sharing_consumers():
     _note("epilogue q only")
     dtype = torch.bfloat16
