@@ -8,17 +8,6 @@
 
 namespace mcamd {
 
-// Sum over the wave, in every lane (a DPP prefix sum's last lane).
-__device__ __forceinline__ int wave_total(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-  return __builtin_amdgcn_readlane(v, 63);
-}
-
 // Block i of a varlen launch of up to 64 sequences, lane b of the wave holding in `mine` how many
 // blocks sequence b has, at most n_qt: the blocks that exist, by their number qt within their
 // sequence, last first (the most keys before the window's edge), a sequence per id within a

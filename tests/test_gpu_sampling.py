@@ -110,3 +110,33 @@ def test_top_k_with_ties_and_a_vocabulary_read_from_memory():
             assert np.array_equal(ids[ok], want[ok]), (V, k)
             kept = np.stack([S.top_k_mask(logits[r].numpy(), k) for r in range(B)])
             assert kept[np.arange(B), ids].all()
+
+
+@pytest.mark.parametrize("V", [3, 4, 5, 1021, 4097, 32768, 32771, 70001])
+@pytest.mark.parametrize("k", [1, 2, 63, 256, 257, 1024, 1025, 5000, "V - 1"])
+def test_top_k_sets_at_the_edges_of_the_search(V, k):
+    """Every way the k-th largest is found: one wave's candidates, more of them, a row whose
+    candidates do not fit (equal logits, k past the thread count); rows with NaN and with all but a
+    few logits masked to -inf; odd rows (16-byte loads at any float)."""
+    k = V - 1 if k == "V - 1" else k
+    if k >= V:
+        pytest.skip("top_k >= vocab draws from the whole row")
+    _note("sampler top_k edges", V, k)
+    g = torch.Generator().manual_seed(11)
+    logits = torch.randn(8, V, generator=g) * 3
+    logits[1] = torch.randint(-3, 4, (V,), generator=g).float()    # ties everywhere
+    logits[2] = 0.25                                               # one value
+    logits[3, torch.randperm(V, generator=g)[: V // 2]] = float("nan")
+    logits[4] = float("-inf")
+    logits[4, torch.randperm(V, generator=g)[:3]] = torch.tensor([1.0, 2.0, 0.5])[:V]
+    logits[5] = torch.linspace(-4, 4, V)                           # the largest in the last threads
+    logits[6] = torch.linspace(4, -4, V)
+    logits[7, 1::2] = torch.finfo(torch.float32).min
+    sampler = PhiloxSampler(8, DEV, base_seed=77)
+    ids = sampler(logits.to(DEV), 0.8, top_k=k).view(-1).cpu().numpy()
+    for r in range(8):
+        row = logits[r].numpy()
+        assert S.top_k_mask(row, k)[ids[r]], r
+        s = S.scores(np.where(np.isnan(row), -np.inf, row), 77 + r, 0, 0.8, None)
+        s = np.where(S.top_k_mask(row, k), s, -np.inf)
+        assert s[ids[r]] >= s.max() - 1e-3, r  # the fp32 evaluation's own near-ties aside
