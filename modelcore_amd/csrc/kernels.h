@@ -64,9 +64,8 @@ int device_cus();
 // (prefill_split.h); 0 where it would not. Without it the call runs uncut.
 size_t prefill_scratch_bytes(const AttnArgs &a);
 
-// Split-K geometry of the decode path: keys per split and the number of splits a row can need.
+// Split-K geometry of the general decode path: keys per split, at most.
 constexpr int kDecodeSplitLen = 256;
-int64_t decode_max_splits(int64_t t_max, int64_t window);
 
 // Workspace of the decode path: scratch for the split partials (and the fused path's per-unit
 // descriptors), written and read within one call; no contents are required on entry.

@@ -1,0 +1,105 @@
+"""The general single-token decode (decode_splitk.hip) at the edges of its splits and chunks, its
+own append, and the bf16 / head_dim 128 decode's merge over very many segments, against the float64
+oracle within the dtype's tolerance. The appended caches are compared bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from _util import ATOL, bits, make_case, max_abs, to_np
+from modelcore_amd.kernels.flash_attn import flash_attn
+from oracle import kv_oracle as ko
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+
+
+def _run(c, window, append=True):
+    g = {k: v.to(DEV) for k, v in c.items()}
+    out = flash_attn.flash_attn_with_kvcache(g["q"], g["k_cache"], g["v_cache"],
+                                             k=g["k"] if append else None,
+                                             v=g["v"] if append else None,
+                                             cache_seqlens=g["cache_seqlens"], causal=True,
+                                             window_size=(window, 0))
+    torch.cuda.synchronize()
+    return out, g
+
+
+def _oracle(c, window, append=True):
+    q, kc, vc = to_np(c["q"]), to_np(c["k_cache"]), to_np(c["v_cache"])
+    k, v = (to_np(c["k"]), to_np(c["v"])) if append else (None, None)
+    return ko.flash_attn_with_kvcache(q, kc, vc, k, v, c["cache_seqlens"].tolist(), window)[0]
+
+
+CASES = [
+    # seqlens, H, H_kv, D, T_max, window
+    ([0, 62, 63, 64, 65, 127, 128], 4, 2, 128, 300, -1),     # fp32: 64-key splits
+    ([0, 127, 128, 255, 256, 257], 6, 6, 64, 300, -1),       # fp32: 128; bf16: one split of 256
+    ([511, 512, 767, 3], 16, 2, 64, 800, -1),                # G = 8: two keys a chunk
+    ([700, 64, 33], 12, 4, 96, 800, 63),                     # padded dims, a window of one split
+    ([500, 1], 16, 1, 256, 600, 300),                        # G = 16: two head chunks append once
+    ([31, 32, 33], 3, 3, 16, 40, -1),
+    ([90, 10], 4, 4, 8, 100, -1),                            # half of each key's two lanes
+    # 2048 workgroups or more: splits of 512 keys
+    ([(37 * i) % 1024 for i in range(64)], 16, 16, 16, 1024, -1),
+    ([1023] + [i % 5 for i in range(63)], 32, 16, 16, 1024, -1),
+]
+
+
+@pytest.mark.parametrize("append", [True, False], ids=["append", "no-append"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("seqlens,H,H_kv,D,T_max,window", CASES)
+def test_split_edges_match_the_oracle(dtype, seqlens, H, H_kv, D, T_max, window, append):
+    print("case: splits", dtype, seqlens[:8], H, H_kv, D, T_max, window, append, flush=True)
+    c = make_case(seqlens, 1, H, H_kv, D, T_max, dtype, seed=51)
+    out, g = _run(c, window, append)
+    assert max_abs(to_np(out), _oracle(c, window, append)) <= ATOL[dtype]
+    want = (bits(c["k_cache"]), bits(c["v_cache"]))
+    if append:
+        want = ko.append(*want, bits(c["k"]), bits(c["v"]), seqlens)
+    assert np.array_equal(bits(g["k_cache"]), want[0]) and np.array_equal(bits(g["v_cache"]), want[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_values_past_the_split_and_infinities(dtype):
+    """Stale keys past a row's end are never used; an infinite last value gives an infinite
+    output although the chunk's missing keys re-read it; rows outside the cache get NaN."""
+    print("case: splits, non-finite", dtype, flush=True)
+    seqlens = [70, 200, 299, 300]
+    c = make_case([70, 200, 299, 0], 1, 4, 2, 64, 300, dtype, seed=52)
+    ref = _oracle(c, -1)
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    c["k_cache"][0, 71:] = float("nan")
+    c["v_cache"][0, 71:] = float("nan")
+    c["v"][1, 0, 0, 7] = float("inf")
+    out, g = _run(c, -1)
+    assert max_abs(to_np(out[0]), ref[0]) <= ATOL[dtype]
+    assert torch.isposinf(out[1, 0, :2, 7]).all() and torch.isfinite(out[1, 0, 2:]).all()
+    assert max_abs(to_np(out[1, 0, :, 8:]), ref[1, 0, :, 8:]) <= ATOL[dtype]
+    assert torch.isnan(out[3]).all()
+    assert torch.equal(g["k_cache"][3].cpu(), c["k_cache"][3])
+
+
+@pytest.mark.parametrize("seqlens,H,H_kv,T_max,window", [
+    ([16000], 32, 8, 16400, -1),       # 128 segments a unit
+    ([2500], 4, 1, 2600, -1),          # one unit over the launch, idle KV rows
+    ([900, 2000, 5], 10, 2, 2100, 1500),
+    ([-1, 3000], 8, 4, 3100, -1),      # a row outside the cache beside one of many segments
+])
+def test_merge_of_very_many_segments(seqlens, H, H_kv, T_max, window):
+    dtype = torch.bfloat16
+    print("case: wide merge", seqlens, H, H_kv, T_max, window, flush=True)
+    c = make_case([max(s, 0) for s in seqlens], 1, H, H_kv, 128, T_max, dtype, seed=53)
+    ref = _oracle(c, window)
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    out, _ = _run(c, window)
+    ok = [i for i, s in enumerate(seqlens) if s >= 0]
+    assert max_abs(to_np(out[ok]), ref[ok]) <= ATOL[dtype]
+    assert torch.isnan(out[[i for i, s in enumerate(seqlens) if s < 0]]).all()
+    sl = c["cache_seqlens"].to(DEV)
+    g = {k: v.to(DEV) for k, v in c.items()}
+    moved = flash_attn.flash_attn_with_kvcache(g["q"], g["k_cache"], g["v_cache"], k=g["k"], v=g["v"],
+                                               cache_seqlens=sl, causal=True,
+                                               window_size=(window, 0), advance=2)
+    assert torch.equal(moved[ok], out[ok])
+    assert torch.equal(sl.cpu(), c["cache_seqlens"] + 2)
