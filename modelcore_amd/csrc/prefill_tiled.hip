@@ -13,7 +13,8 @@
 // they take the same 32 pairs and a quarter of each staged tile each, and merge at the end; four
 // times the workgroups and a quarter of the serial chain, for calls with too few pairs to fill the
 // chip (each K/V byte is then staged for a quarter of the pairs). Blocks with the most keys (the
-// last positions) are launched first.
+// last positions) are launched first; a compute unit holds two or three at once, so they are dealt to
+// the compute units there and back (dealt_block()).
 //
 // Products, per wave and 32 keys, with both 32 x 32 results transposed so that a lane owns one
 // pair (lane l: pair l % 32, keys 8j + 4(l / 32) + i):
@@ -28,9 +29,9 @@
 //    8c + 4 + i, so that a lane reads its K row as 16-byte vectors.
 //
 // Measured against the VALU kernel this replaced (four lanes a row, an LDS float per FMA): four
-// 2048-token prompts of 12 heads of 64 in bf16 1858 -> 66 us (390 TFLOP/s of the attended pairs;
-// bound by the weights' exponentials and conversions on the VALU), in fp32 287 us (90 of the 144
-// TFLOP/s a large fp32 product reaches); two of 512 tokens in fp32 192 -> 30 us.
+// 2048-token prompts of 12 heads of 64 in bf16 1858 -> 64 us (400 TFLOP/s of the attended pairs;
+// bound by the weights' exponentials and conversions on the VALU), in fp32 262 us (98 of the 154
+// TFLOP/s a large fp32 product reaches); two of 512 tokens in fp32 192 -> 29 us.
 //
 // Online softmax per pair in fp32 (exp2 domain): weights are made against the running maximum, and
 // the tile's own maximum is taken (and O rescaled) only when a lane's weights of the tile sum past
@@ -70,6 +71,7 @@ struct TiledParams {
   const int32_t *rows, *cu;  // varlen (optional): cache row and token range per sequence
   void *out;
   int T_new, H, H_kv, G, T_max, window, D, n_bh, n_qt;
+  int deal;  // workgroups per round of dealt_block()
   int64_t cache_b;
   float scale_log2;
   SplitGeo split;
@@ -183,9 +185,10 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   E *const sK = reinterpret_cast<E *>(s_raw);
   E *const sV = sK + KT * KSTR;
 
-  int bh = blockIdx.x % P.n_bh;
-  const int part = int(blockIdx.x / P.n_bh) % P.split.n_split;  // key range
-  int qt = P.n_qt - 1 - int(blockIdx.x / P.n_bh) / P.split.n_split;
+  const int id = P.cu ? int(blockIdx.x) : dealt_block(int(blockIdx.x), int(gridDim.x), P.deal);
+  int bh = id % P.n_bh;
+  const int part = int(id / P.n_bh) % P.split.n_split;  // key range
+  int qt = P.n_qt - 1 - int(id / P.n_bh) / P.split.n_split;
   int b = bh / P.H_kv;
   int kvh = bh - b * P.H_kv;
   int row = b, T_b = P.T_new, s0;
@@ -403,14 +406,17 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
             __builtin_convertvector(pv - __builtin_convertvector(hi8, f32x8), bf16x8);
         const uint16_t *vp = reinterpret_cast<const uint16_t *>(sV) +
                              (wk + 16 * ks + 4 * h + tr_row) * VSTR + tr_col;
+        bf16x8 a[MD];  // the lo terms after all hi terms: no product waits for the one before it
 #pragma unroll
         for (int md = 0; md < MD; ++md) {
           const bf16x4 a0 = lds_read_tr(vp + 32 * md);
           const bf16x4 a1 = lds_read_tr(vp + 8 * VSTR + 32 * md);
-          const bf16x8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-          o[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, hi8, o[md], 0, 0, 0);
-          o[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, lo8, o[md], 0, 0, 0);
+          a[md] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+          o[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[md], hi8, o[md], 0, 0, 0);
         }
+#pragma unroll
+        for (int md = 0; md < MD; ++md)
+          o[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[md], lo8, o[md], 0, 0, 0);
       }
     } else {
       const float *vp = reinterpret_cast<const float *>(sV) + (wk + 4 * h) * VSTR + col;
@@ -633,6 +639,7 @@ TiledParams tiled_params(const AttnArgs &a) {
   P.D = int(a.head_dim);
   P.n_bh = int(a.batch * a.n_kv_head);
   P.n_qt = 0;
+  P.deal = device_cus();
   P.cache_b = a.cache_batch_stride;
   P.scale_log2 = float(kLog2e / std::sqrt(double(a.head_dim)));
   P.split = SplitGeo{};

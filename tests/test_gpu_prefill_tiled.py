@@ -73,6 +73,17 @@ def test_tile_edges_match_the_oracle(dtype, seqlens, T_new, H, H_kv, D, T_max, w
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,T_new,heads", [(7, 129, 19), (3, 65, 29), (5, 129, 64), (1, 33, 131)],
+                         ids=["pairs-266", "keys-261", "pairs-640", "keys-262"])
+def test_every_block_of_more_than_one_round_of_workgroups_is_written(dtype, rows, T_new, heads):
+    """Blocks past the first 256 are dealt the other way round in steps of 8, with a rest."""
+    print("case: tiled rounds", dtype, rows, T_new, heads, flush=True)
+    c = make_case([11 * b for b in range(rows)], T_new, heads, heads, 32, T_new + 11 * rows, dtype,
+                  seed=43)
+    _close(_run(c, -1), _oracle(c, -1), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads", [2, 128], ids=["keys-over-waves", "pairs-over-waves"])
 def test_infinities_and_nan_reach_only_the_pairs_that_see_them(dtype, heads):
     """Values past a query's position are multiplied by a weight of zero on the matrix cores: a
