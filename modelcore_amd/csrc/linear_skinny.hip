@@ -16,10 +16,12 @@
 // fixed order, so results never depend on timing (nor on the tile shape: a partial's k order is
 // the same).
 //
+// The gated product runs unsplit with eight, four or two waves (launch_gated()).
+//
 // Data path. The K-range is walked in stages of 128: one stage is 16 WAVES rows x 256 bytes of W
 // and 64 rows x 256 bytes of x, brought into LDS by buffer_load ... lds (16 bytes per lane, four
 // rows of 256 contiguous bytes per instruction, so every HBM line is read whole), RING - 1
-// stages ahead in a ring of RING (4 with four waves, 3 with eight: 128 and 144 KB of LDS). Each
+// stages ahead in a ring of RING (4 with two or four waves, 3 with eight: 96, 128 and 144 KB of LDS). Each
 // wave moves its own 16 rows of W and a share of x. W is loaded non-temporal (read once: its
 // lines should not push the activations out of L2). The buffer resources bound every read (rows
 // of x past M read as zero). In LDS a row keeps its sixteen 16-byte chunks, chunk c of row r at
@@ -50,8 +52,7 @@ struct LinParams {
   int64_t ldx, ldy;
   int M, N, K, S;
   int raw;      // write the partials (fp32) even for S = 1, and leave the sum to the consumer
-  int gated;    // W holds [gate; up] interleaved in 64-row blocks: write silu(gate) * up to y
-  int w_tiled;  // W stored as (N / 64, K / 128, 64, 128) blocks instead of row-major (N, K)
+  int w_tiled;  // gated: W stored as (N / 64, K / 128, 64, 128) blocks instead of row-major (N, K)
 };
 
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
@@ -107,7 +108,9 @@ __device__ __forceinline__ uint16_t silu_mul_bf16(float gate, float up) {
 // The leading arguments repeat the fields of P that the tile set-up needs, so that they arrive
 // preloaded in SGPRs at dispatch (the library is built with kernarg preloading, which covers
 // scalar arguments only) rather than through a load from the kernel-argument buffer.
-template <int WAVES, int MB>  // MB blocks of 16 activation rows: M <= 16 MB
+// GATED: W holds [gate; up] interleaved in 64-row blocks; silu(gate) * up goes to y. Wave w of the
+// launch owns hidden units 8 w .. 8 w + 7, its 16 rows being their gate rows and then their up rows.
+template <int WAVES, int MB, bool GATED>  // MB blocks of 16 activation rows: M <= 16 MB
 __global__ __launch_bounds__(64 * WAVES, 1) void linear_skinny_kernel(
     const uint16_t *a_x, const uint16_t *a_w, int64_t a_ldx, int a_M, int a_N, int a_K, int a_S,
     int a_w_tiled, LinParams P) {
@@ -134,9 +137,12 @@ __global__ __launch_bounds__(64 * WAVES, 1) void linear_skinny_kernel(
   const int k_begin = blockIdx.y * ks;
   const int stages = ks / KC;
 
-  const uint32_t wbytes = uint32_t(min(kRows, P.N - n0)) * uint32_t(P.K) * 2u;
+  // W rows of this workgroup; gated: of the 128-row block pair that holds this wave's units.
+  const int unit = int(blockIdx.x) * WAVES + wave;  // of 8 hidden units; they are a multiple of WAVES
+  const int w0 = GATED ? unit / 8 * 128 : n0;
+  const uint32_t wbytes = uint32_t(GATED ? 128 : min(kRows, P.N - n0)) * uint32_t(P.K) * 2u;
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)(P.w + int64_t(n0) * P.K), 0, int(wbytes), 0x00020000);
+      (void *)(P.w + int64_t(w0) * P.K), 0, int(wbytes), 0x00020000);
   const uint32_t xbytes = uint32_t(P.M) * uint32_t(P.ldx) * 2u;
   const __amdgpu_buffer_rsrc_t rx =
       __builtin_amdgcn_make_buffer_rsrc((void *)P.x, 0, int(xbytes), 0x00020000);
@@ -153,12 +159,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void linear_skinny_kernel(
       const int r0 = 4 * (4 * wave + jj);
       const int r = r0 + drow;
       const uint32_t chunk = uint32_t(dslot ^ (r & 15));
-      // Row-major: row r of the tile, bytes kb .. kb + 255. Tiled: the tile's 64-row group
-      // r / 64 (K * 128 bytes each, at the same place as in row-major), its 16 KB block of this
-      // stage, row r % 64 of the block -- an instruction reads 1 KB contiguous.
-      const uint32_t wo = P.w_tiled ? uint32_t(r >> 6) * uint32_t(P.K) * 128u + kb * 64u +
-                                          uint32_t(r & 63) * 256u + chunk * 16u
-                                    : uint32_t(r) * uint32_t(P.K) * 2u + kb + chunk * 16u;
+      // Row-major: row src of the tile, bytes kb .. kb + 255. Tiled: its 64-row group src / 64 (K * 128
+      // bytes each, at the same place as in row-major), its 16 KB block of this stage, row src % 64 of
+      // the block -- an instruction reads 1 KB contiguous.
+      const int src = GATED ? 64 * (jj >> 1) + unit % 8 * 8 + 4 * (jj & 1) + drow : r;
+      const uint32_t wo = GATED && P.w_tiled
+                              ? uint32_t(src >> 6) * uint32_t(P.K) * 128u + kb * 64u +
+                                    uint32_t(src & 63) * 256u + chunk * 16u
+                              : uint32_t(src) * uint32_t(P.K) * 2u + kb + chunk * 16u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rw, (__attribute__((address_space(3))) void *)(&sW[buf][r0 * KC]), 16, int(wo), 0, 0,
           kNonTemporal);
@@ -238,36 +246,27 @@ __global__ __launch_bounds__(64 * WAVES, 1) void linear_skinny_kernel(
   }
 
   // acc[mb][i] = y[m = 16 mb + l % 16][n = n0 + 16 w + 4 (l / 16) + i].
-  if constexpr (WAVES == 8) {
-    if (P.gated) {
-      // Rows 0..63 of the tile are gate rows j, rows 64..127 the up rows of the same j: wave
-      // w + 4 holds, lane for lane, the up values of wave w's gate values. They pass through
-      // LDS (the W ring, free once every wave is past its last stage: a full __syncthreads, so
-      // that no store below can be moved above it).
-      float *xch = reinterpret_cast<float *>(&sW[0][0]);
-      __syncthreads();
-      if (wave >= 4) {
+  if constexpr (GATED) {
+    // Lanes 0..31 hold gate values, lanes 32..63, row for row, the up values of the same units. Two
+    // blocks of activation rows change halves: the first then has its products in lanes 0..31, the
+    // second in 32..63 (an odd last block changes with itself).
+    const int j = 8 * unit + 4 * (fq & 1);  // hidden unit of acc[.][0]
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < MB; mb += 2) {
+      const int m = 16 * (mb + (lane >> 5)) + fr;
+      uint16_t hv[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) xch[(((wave - 4) * MB + mb) * 4 + i) * 64 + lane] = acc[mb][i];
+      for (int i = 0; i < 4; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(acc[mb][i]), __float_as_uint(acc[mb + 1 < MB ? mb + 1 : mb][i]), false,
+            false);
+        hv[i] = silu_mul_bf16(__uint_as_float(r[0]), __uint_as_float(r[1]));
       }
-      __syncthreads();
-      if (wave >= 4) return;
-      const int j = blockIdx.x * 64 + 16 * wave + 4 * fq;  // hidden unit of acc[.][0]
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const int m = 16 * mb + fr;
-        if (m >= P.M) continue;
-        uint16_t hv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          hv[i] = silu_mul_bf16(acc[mb][i], xch[((wave * MB + mb) * 4 + i) * 64 + lane]);
+      if (m < P.M && mb + (lane >> 5) < MB)
         *reinterpret_cast<uint2 *>(P.y + int64_t(m) * P.ldy + j) =
             uint2{uint32_t(hv[0]) | (uint32_t(hv[1]) << 16), uint32_t(hv[2]) | (uint32_t(hv[3]) << 16)};
-      }
-      return;
     }
+    return;
   }
   const int n = n0 + 16 * wave + 4 * fq;
   if (n >= P.N) return;
@@ -299,18 +298,21 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinParams P) {
   *reinterpret_cast<uint2 *>(P.y + m * P.ldy + n) = uint2{lo, hi};
 }
 
-template <int WAVES>
+template <int WAVES, bool GATED>
 void launch_skinny(const LinParams &P, hipStream_t s) {
   const dim3 grid(unsigned((P.N + 16 * WAVES - 1) / (16 * WAVES)), unsigned(P.S));
   const dim3 block(64 * WAVES);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, P.x, P.w, P.ldx, P.M, P.N, P.K, P.S, P.w_tiled, P);
+  };
   if (P.M <= 16)
-    hipLaunchKernelGGL((linear_skinny_kernel<WAVES, 1>), grid, block, 0, s, P.x, P.w, P.ldx, P.M, P.N, P.K, P.S, P.w_tiled, P);
+    launch(linear_skinny_kernel<WAVES, 1, GATED>);
   else if (P.M <= 32)
-    hipLaunchKernelGGL((linear_skinny_kernel<WAVES, 2>), grid, block, 0, s, P.x, P.w, P.ldx, P.M, P.N, P.K, P.S, P.w_tiled, P);
+    launch(linear_skinny_kernel<WAVES, 2, GATED>);
   else if (P.M <= 48)
-    hipLaunchKernelGGL((linear_skinny_kernel<WAVES, 3>), grid, block, 0, s, P.x, P.w, P.ldx, P.M, P.N, P.K, P.S, P.w_tiled, P);
+    launch(linear_skinny_kernel<WAVES, 3, GATED>);
   else
-    hipLaunchKernelGGL((linear_skinny_kernel<WAVES, 4>), grid, block, 0, s, P.x, P.w, P.ldx, P.M, P.N, P.K, P.S, P.w_tiled, P);
+    launch(linear_skinny_kernel<WAVES, 4, GATED>);
 }
 
 }  // namespace
@@ -365,9 +367,25 @@ void launch_linear(const LinParams &P, hipStream_t s) {
   const bool wide = P.S == 1 && P.N >= 192 * 128;
   const bool split128 = P.S > 1 && P.N % 128 == 0 && int64_t(P.N / 128) * P.S <= 256;
   if (P.M > 16 && (wide || split128))
-    launch_skinny<8>(P, s);
+    launch_skinny<8, false>(P, s);
   else
-    launch_skinny<4>(P, s);
+    launch_skinny<4, false>(P, s);
+}
+
+// Eight waves a workgroup (64 hidden units), or half or a quarter of them while twice the workgroups
+// still fit one per compute unit: narrower MLPs left half the chip and more idle. A captured decode block,
+// eight waves against this rule: 2048 wide with 8192 hidden units (four waves) 3 rows 62.7 against 59.4 us, 30
+// rows 79.2 / 74.3, 64 rows 93.7 / 87.6; 1536 wide with 4096 (two) 3 rows 53.7 / 49.8, 64 rows 76.7 / 72.8 (four:
+// 51.5 and 74.2). 14336 stays at eight: 134 us, four 141 (every workgroup reads all of x), seven, which give
+// 256 even workgroups instead of 224, 134.
+void launch_gated(const LinParams &P, hipStream_t s) {
+  const int64_t units = P.N / 16, cus = device_cus();
+  if (units / 8 * 2 > cus)
+    launch_skinny<8, true>(P, s);
+  else if (units / 4 * 2 > cus)
+    launch_skinny<4, true>(P, s);
+  else
+    launch_skinny<2, true>(P, s);
 }
 
 }  // namespace
@@ -420,9 +438,8 @@ extern "C" int mcamd_linear_bf16_gated(const void *x, int64_t ldx, const void *w
     return fail(MCAMD_EINVAL, "linear_bf16_gated: need h with ldh >= hidden (a multiple of 4)");
   P.y = static_cast<uint16_t *>(h);
   P.ldy = ldh;
-  P.gated = 1;
   P.w_tiled = w_tiled != 0;
-  launch_skinny<8>(P, as_stream(stream));  // a 128-row tile holds 64 gate and their 64 up rows
+  launch_gated(P, as_stream(stream));
   return launch_status("linear_bf16_gated");
 }
 

@@ -80,7 +80,10 @@ def test_unsupported_shapes_are_refused():
 
 
 @pytest.mark.parametrize("tiled", [False, True], ids=["row-major", "tiled"])
-@pytest.mark.parametrize("m,hid,k", [(64, 14336, 4096), (5, 768, 384), (64, 128, 1024)])
+@pytest.mark.parametrize("m,hid,k", [(64, 14336, 4096), (5, 768, 384), (64, 128, 1024),
+                                     # the widest of two, four and the narrowest of eight waves
+                                     (33, 8256, 256), (17, 8192, 256), (48, 4160, 128), (64, 4096, 256),
+                                     (1, 64, 128)])
 def test_gated_silu_product_matches_the_separate_bf16_ops(m, hid, k, tiled):
     """linear_bf16_gated on the interleaved [W_gate; W_up] against torch's silu(g) * u of the
     kernel's own bf16 products g = x W_gate^T, u = x W_up^T (one K split, so the same fp32 sums):
