@@ -5,11 +5,10 @@
 // which is both the sliced uniform path (:217-224) and the ragged mask (:246-264). Query head h
 // reads KV head h / G, G = H / H_kv (SDPA enable_gqa). Scale 1/sqrt(D).
 //
-// Work split. The key range of a row is cut into splits of up to kDecodeSplitLen keys, aligned to
-// lo. One workgroup owns (row b, KV head, split) and serves every query head of that KV head's GQA
-// group (up to GM at a time), so each K/V byte of the split is read from HBM once. The grid is
-// sized from T_max (no host sync on cache_seqlens); splits past a row's length exit at once. Small
-// calls take shorter splits, so that more workgroups share the wait for memory (decode_split_len).
+// Work split. The key range of a row is cut into splits, aligned to lo. One workgroup owns (row b,
+// KV head, split) and serves every query head of that KV head's GQA group (up to GM at a time), so
+// each K/V byte of the split is read from HBM once. The grid is sized from T_max (no host sync on
+// cache_seqlens); splits past a row's length exit at once. The length of a split: decode_split.h.
 //
 // Inside a workgroup (256 threads): LPT = DP / VEC lanes cover one key's D elements with one
 // 16-byte load each, so a wave reads 64/LPT whole head rows per instruction, and each group of LPT
@@ -29,6 +28,7 @@
 // 256-4096 keys, 16 / 4 heads of 128 in fp32 (286 MB) 62 (92). Before, each split read K, stored its
 // scores in LDS, took the softmax there and read V after it, with the append and the merge as
 // launches of their own.
+#include "decode_split.h"
 #include "kernels.h"
 
 #include <cmath>
@@ -386,12 +386,6 @@ int dispatch_d(DecodeParams &P, int B, hipStream_t s) {
 
 namespace {
 
-int64_t span_of(int64_t t_max, int64_t window) {
-  return window >= 0 ? std::min<int64_t>(t_max, window + 1) : t_max;
-}
-int64_t splits_of(int64_t t_max, int64_t window, int64_t len) {
-  return (span_of(t_max, window) + len - 1) / len;
-}
 size_t general_bytes(int64_t batch, int64_t n_head, int64_t head_dim, int64_t splits) {
   return size_t(batch * n_head * splits * (head_dim + 2) * 4);
 }
@@ -402,30 +396,12 @@ size_t short_split_room(int64_t batch, int64_t n_head, int64_t n_kv_head, int64_
                          : size_t(4) << 20;
 }
 
-// Keys per split: kDecodeSplitLen, or less where even a full cache gives few workgroups, down to
-// 32 KB of keys (two rows' chunks in flight are 16 KB each). A pure function of the sizes: every
-// entry point gives the same sums. Measured, shorter against 256 keys, with the merge: 16 query / 2 KV
-// heads of 128 in fp32, one row of 4000 keys 26.4 against 35.8 us; 8 heads of 256 in fp32, one row of
-// 300 keys 10.2 against 16.6; but 12 heads of 64 in bf16 (32 KB are 256 keys), one row of 2000 keys,
-// 11.0 at 64 keys against 8.5. Longer where they are many: 32 rows of 512-8192 keys, 16 / 4 heads of 64
-// in bf16, 512 keys 41.7 us against 47.7 at 256 (1024 keys 39.0, but 20 KV heads' worth of shorter rows
-// lose up to 40% at so few workgroups).
 int64_t decode_split_len(int64_t batch, int64_t n_head, int64_t n_kv_head, int64_t head_dim,
                          int64_t t_max, int64_t window, int64_t elem) {
-  int64_t len = 64;
-  while (len < kDecodeSplitLen && len * head_dim * elem < 32768) len *= 2;
-  for (; len < kDecodeSplitLen; len *= 2) {
-    const int64_t ns = splits_of(t_max, window, len);
-    if (ns <= 64 && batch * n_kv_head * ns <= 1024 &&
-        general_bytes(batch, n_head, head_dim, ns) <=
-            short_split_room(batch, n_head, n_kv_head, head_dim, t_max, window))
-      return len;
-  }
-  // Longer while that leaves 2048 workgroups (eight per compute unit).
-  int64_t len_up = kDecodeSplitLen;
-  while (len_up < 2048 && batch * n_kv_head * splits_of(t_max, window, 2 * len_up) >= 2048)
-    len_up *= 2;
-  return len_up;
+  return split_len(batch, n_kv_head, head_dim, t_max, window, elem, [&](int64_t splits) {
+    return general_bytes(batch, n_head, head_dim, splits) <=
+           short_split_room(batch, n_head, n_kv_head, head_dim, t_max, window);
+  });
 }
 
 }  // namespace

@@ -64,9 +64,6 @@ int device_cus();
 // (prefill_split.h); 0 where it would not. Without it the call runs uncut.
 size_t prefill_scratch_bytes(const AttnArgs &a);
 
-// Split-K geometry of the general decode path: keys per split, at most.
-constexpr int kDecodeSplitLen = 256;
-
 // Workspace of the decode path: scratch for the split partials (and the fused path's per-unit
 // descriptors), written and read within one call; no contents are required on entry.
 size_t decode_workspace_bytes(int64_t batch, int64_t n_head, int64_t n_kv_head, int64_t head_dim,

@@ -40,7 +40,7 @@ CASES = [
     ([500, 1], 16, 1, 256, 600, 300),                        # G = 16: two head chunks append once
     ([31, 32, 33], 3, 3, 16, 40, -1),
     ([90, 10], 4, 4, 8, 100, -1),                            # half of each key's two lanes
-    # 2048 workgroups or more: splits of 512 keys
+    # 64 rows of four splits each at most, most of them shorter
     ([(37 * i) % 1024 for i in range(64)], 16, 16, 16, 1024, -1),
     ([1023] + [i % 5 for i in range(63)], 32, 16, 16, 1024, -1),
 ]
@@ -103,3 +103,21 @@ def test_merge_of_very_many_segments(seqlens, H, H_kv, T_max, window):
                                                window_size=(window, 0), advance=2)
     assert torch.equal(moved[ok], out[ok])
     assert torch.equal(sl.cpu(), c["cache_seqlens"] + 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T_max,length", [(1024, 512), (2048, 1024), (4096, 2048)])
+def test_long_splits_of_large_grids(dtype, T_max, length):
+    """4096 (row, KV head)s of two splits: three rows at a split's edges against the oracle."""
+    print("case: long splits", dtype, T_max, length, flush=True)
+    B, H, D = 64, 64, 16 // dtype.itemsize
+    seqlens = [(97 * b) % T_max for b in range(B)]
+    seqlens[:4] = [length - 1, length, T_max - 1, length // 2]
+    g = torch.Generator(device=DEV).manual_seed(54)
+    c = {n: torch.randn(B, T, H, D, generator=g, device=DEV).to(dtype)
+         for n, T in (("q", 1), ("k", 1), ("v", 1), ("k_cache", T_max), ("v_cache", T_max))}
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32, device=DEV)
+    rows = {n: t[:4].clone() for n, t in c.items()}
+    out, _ = _run(c, -1)
+    assert max_abs(to_np(out[:4]), _oracle(rows, -1)) <= ATOL[dtype]
+    assert torch.isfinite(out).all()
