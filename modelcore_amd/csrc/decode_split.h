@@ -11,6 +11,7 @@ constexpr int64_t kDecodeSplitLen = 256;
 // Workgroups that remain where splits are made longer than that, and how long they get.
 constexpr int64_t kLongSplitBlocks = 8192;
 constexpr int64_t kLongestSplit = 2048;
+constexpr int64_t kMostSplits = 65535;  // a grid's blocks along y
 
 // Keys a row can attend, and its splits of `len` keys.
 inline int64_t span_of(int64_t t_max, int64_t window) {
@@ -46,6 +47,7 @@ int64_t split_len(int64_t batch, int64_t n_kv_head, int64_t head_dim, int64_t t_
   while (len < kLongestSplit &&
          batch * n_kv_head * splits_of(t_max, window, 2 * len) >= kLongSplitBlocks)
     len *= 2;
+  while (splits_of(t_max, window, len) > kMostSplits) len *= 2;
   return len;
 }
 

@@ -121,3 +121,19 @@ def test_long_splits_of_large_grids(dtype, T_max, length):
     out, _ = _run(c, -1)
     assert max_abs(to_np(out[:4]), _oracle(rows, -1)) <= ATOL[dtype]
     assert torch.isfinite(out).all()
+
+
+def test_a_cache_of_more_positions_than_a_grid_has_blocks_of_2048():
+    print("case: 135M positions", flush=True)
+    T_max, D = 135_000_000, 8
+    c = {n: torch.zeros(1, T, 1, D, dtype=torch.bfloat16, device=DEV)
+         for n, T in (("q", 1), ("k", 1), ("v", 1), ("k_cache", T_max), ("v_cache", T_max))}
+    g = torch.Generator(device=DEV).manual_seed(55)
+    for n in ("q", "k", "v"):
+        c[n].normal_(generator=g)
+    for n in ("k_cache", "v_cache"):
+        c[n][:, :5000].normal_(generator=g)
+    c["cache_seqlens"] = torch.tensor([4999], dtype=torch.int32, device=DEV)
+    small = {n: t[:, :5000].clone() if n.endswith("cache") else t for n, t in c.items()}
+    out, _ = _run(c, -1)
+    assert max_abs(to_np(out), _oracle(small, -1)) <= ATOL[torch.bfloat16]

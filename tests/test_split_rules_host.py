@@ -4,6 +4,8 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import pytest
+
 CSRC = Path(__file__).resolve().parent.parent / "modelcore_amd" / "csrc"
 
 SPLIT_LEN = """
@@ -47,3 +49,10 @@ def test_rows_shorter_than_their_cache_keep_their_decode_workgroups(tmp_path):
             assert b * h * -(-span // n) >= 8192, (b, h, d, t, w, e, n)
         # Rows of an eighth of the cache's length: a workgroup per compute unit, or 256 keys each.
         assert n <= 256 or b * h * -(-(span // 8) // n) >= 256, (b, h, d, t, w, e, n)
+
+
+@pytest.mark.parametrize("t_max", [(1 << 24) + 1, 135_000_000, 1 << 30])
+def test_decode_splits_fit_a_grid(tmp_path, t_max):
+    cases = [(b, h, 8, t_max, -1, e) for b in (1, 5, 64) for h in (1, 8) for e in (2, 4)]
+    for n in _split_lens(tmp_path, cases):
+        assert -(-t_max // n) <= 65535
