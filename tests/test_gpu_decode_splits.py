@@ -137,3 +137,24 @@ def test_a_cache_of_more_positions_than_a_grid_has_blocks_of_2048():
     small = {n: t[:, :5000].clone() if n.endswith("cache") else t for n, t in c.items()}
     out, _ = _run(c, -1)
     assert max_abs(to_np(out), _oracle(small, -1)) <= ATOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 256), (torch.float32, 128), (torch.float32, 256)])
+@pytest.mark.parametrize("T_max", [1025, 1300], ids=["odd", "even"])
+def test_paired_splits_of_wide_rows(dtype, D, T_max):
+    """2048 workgroups or more of 512-byte or 1 KB rows: two splits of a head beside each other, an
+    odd and an even number of them."""
+    print("case: paired splits", dtype, D, T_max, flush=True)
+    B, H, H_kv = 64, 16, 8
+    seqlens = [(129 * b) % T_max for b in range(B)]
+    seqlens[:5] = [255, 256, 511, T_max - 1, 0]
+    g = torch.Generator(device=DEV).manual_seed(56)
+    c = {n: torch.randn(B, T, h, D, generator=g, device=DEV).to(dtype)
+         for n, T, h in (("q", 1, H), ("k", 1, H_kv), ("v", 1, H_kv), ("k_cache", T_max, H_kv),
+                         ("v_cache", T_max, H_kv))}
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32, device=DEV)
+    pick = [0, 1, 2, 3, 4, 13, 63]
+    rows = {n: t[pick].clone() for n, t in c.items()}
+    out, _ = _run(c, -1)
+    assert max_abs(to_np(out[pick]), _oracle(rows, -1)) <= ATOL[dtype]
+    assert torch.isfinite(out).all()
