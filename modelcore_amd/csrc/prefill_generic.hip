@@ -126,6 +126,7 @@ __global__ __launch_bounds__(kThreads) void prefill_generic_kernel(PrefillParams
 
     float sc[KT];
     float mt = -INFINITY;
+    bool any = false;  // a key with a weight, or a NaN score, which the maximum passes over
 #pragma unroll
     for (int kk = 0; kk < KT; ++kk) {
       float s = 0.f;
@@ -137,8 +138,9 @@ __global__ __launch_bounds__(kThreads) void prefill_generic_kernel(PrefillParams
       const bool ok = active && col <= p && (P.window < 0 || p - col <= P.window);
       sc[kk] = ok ? s : -INFINITY;
       mt = fmaxf(mt, sc[kk]);
+      any = any || sc[kk] != -INFINITY;
     }
-    if (mt > -INFINITY) {
+    if (any) {
       const float m_new = fmaxf(m, mt);
       const float corr = fast_exp2(m - m_new);
       l *= corr;
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(kThreads) void prefill_generic_kernel(PrefillParams
       for (int i = 0; i < DS; ++i) o[i] *= corr;
 #pragma unroll
       for (int kk = 0; kk < KT; ++kk) {
-        if (sc[kk] > -INFINITY) {
+        if (sc[kk] != -INFINITY) {
           const float pk = fast_exp2(sc[kk] - m_new);
           l += pk;
 #pragma unroll

@@ -148,7 +148,11 @@ __device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at,
       if (d < D) s = fmaf(qv[i], to_f32<E>(kc[int64_t(t) * tok + d]), s);
     }
     s = wave_sum<64>(s);
-    if (!(s > -INFINITY)) continue;
+    if (s == -INFINITY) continue;
+    if (s != s) {  // a key the pair sees makes its output NaN, as in the softmax
+      l = s;
+      break;
+    }
     const float m_new = fmaxf(m, s);
     const float corr = fast_exp2(m - m_new), w = fast_exp2(s - m_new);
     m = m_new;

@@ -109,6 +109,30 @@ def test_infinities_and_nan_reach_only_the_pairs_that_see_them(dtype, heads):
     assert torch.equal(out[3], plain[3])
 
 
+@pytest.mark.parametrize("seqlens,T_new,H,H_kv,D,T_max", [
+    ([40, 3], 40, 2, 2, 64, 100),         # the waves over a block's keys
+    ([40, 3], 40, 512, 128, 64, 100),     # over its pairs
+    ([3000, 1000], 40, 4, 2, 96, 3100),   # key ranges
+    ([40, 3], 40, 2, 2, 384, 100),        # head dims above 256
+    ([3000, 1000], 40, 4, 2, 128, 3100),  # bf16: prefill_mfma.hip
+], ids=["keys", "pairs", "ranges", "wide", "hd128"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_nan_key_makes_every_output_that_sees_it_nan(dtype, seqlens, T_new, H, H_kv, D, T_max):
+    """As the softmax over its scores does; the keys before it, and other KV heads, keep theirs."""
+    print("case: NaN keys", dtype, seqlens, T_new, H, H_kv, D, T_max, flush=True)
+    c = make_case(seqlens, T_new, H, H_kv, D, T_max, dtype, seed=46)
+    good = _run(c, -1)
+    G = H // H_kv
+    c["k"][0, 17, 0, 1] = float("nan")                 # a new key: seen by queries 17.. of row 0
+    c["k_cache"][1, 2, H_kv - 1, 0] = float("nan")     # a cached one: seen by all of row 1
+    out = _run(c, -1)
+    assert torch.isnan(out[0, 17:, :G]).all()
+    _close(out[0, :17], to_np(good[0, :17]), dtype)
+    assert torch.equal(out[0, :, G:], good[0, :, G:])
+    assert torch.isnan(out[1, :, H - G:]).all()
+    assert torch.equal(out[1, :, :H - G], good[1, :, :H - G])
+
+
 SPLIT_CASES = [
     # seqlens, T_new, H, H_kv, D, T_max, window
     ([8000], 100, 32, 8, 128, 8200, -1),          # two blocks of queries, many ranges
