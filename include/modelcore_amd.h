@@ -93,11 +93,10 @@ size_t mcamd_attn_workspace_bytes(int64_t batch, int64_t t_new, int64_t n_head,
                                   int64_t window);
 
 /*
- * Bytes of scratch with which the operator runs these sizes best. t_new == 1: what
- * mcamd_attn_workspace_bytes() gives. t_new > 1, where no workspace is needed: room for the fp32
- * partials of a call with too few queries to fill the GPU, whose keys are then cut into ranges
- * (another order of the same fp32 sums); without it, or with less, such a call runs uncut. 0 where
- * none is of use.
+ * Bytes of scratch with which mcamd_flash_attn_with_kvcache_scratch() runs these sizes best.
+ * t_new == 1: what mcamd_attn_workspace_bytes() gives. t_new > 1, where no workspace is needed: room
+ * for the fp32 partials of a call with too few queries to fill the GPU, whose keys are then cut into
+ * ranges; with less, such a call runs uncut. 0 where none is of use.
  */
 size_t mcamd_attn_scratch_bytes(int64_t batch, int64_t t_new, int64_t n_head, int64_t n_kv_head,
                                 int64_t head_dim, int64_t t_max, int64_t window, int dtype);
@@ -107,7 +106,8 @@ size_t mcamd_attn_scratch_bytes(int64_t batch, int64_t t_new, int64_t n_head, in
  * NULL = no append), then attention of q over the cache under the rules at the top of this
  * file. t_new == 1 runs split-K flash-decoding; t_new > 1 runs chunked prefill against the
  * cache prefix. cache_seqlens is read, never advanced. `causal` is accepted for signature
- * parity and ignored: the path is always causal.
+ * parity and ignored: the path is always causal. The workspace is scratch of t_new == 1 alone
+ * (mcamd_attn_workspace_bytes()): with t_new > 1 it is neither read nor written.
  * Replaces flash_attn_with_kvcache (modelcore/kernels/flash_attn.py:306-366; the FA3 call at
  * :324-328 and the SDPA fallback at :330-366).
  */
@@ -157,6 +157,22 @@ int mcamd_flash_attn_with_kvcache_ex(const void *q, const void *k, const void *v
                                      void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * mcamd_flash_attn_with_kvcache_ex, except that a call with t_new > 1 uses its scratch: with
+ * mcamd_attn_scratch_bytes() of it (16-byte aligned; MCAMD_EINVAL otherwise) a call with few queries
+ * against many keys cuts the keys into ranges that run side by side, whose fp32 partials go to the
+ * scratch. Its outputs are those of the call without scratch in another order of the same sums,
+ * within the dtype's rounding. The scratch belongs to the call until it ends on the stream: calls that
+ * can overlap need one each. With t_new == 1, the same as mcamd_flash_attn_with_kvcache_ex.
+ */
+int mcamd_flash_attn_with_kvcache_scratch(const void *q, const void *k, const void *v,
+                                          void *k_cache, void *v_cache, int32_t *cache_seqlens,
+                                          void *out, int64_t batch, int64_t t_new, int64_t n_head,
+                                          int64_t n_kv_head, int64_t head_dim, int64_t t_max,
+                                          int64_t cache_batch_stride, int64_t window, int causal,
+                                          int dtype, int32_t advance, int64_t shared_prefix,
+                                          void *scratch, size_t scratch_bytes, void *stream);
+
+/*
  * mcamd_flash_attn_with_kvcache without the workspace arguments, for callers that cannot allocate
  * device memory (code under graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * It has no counterpart in the reference. Its scratch is a static device array of
@@ -164,8 +180,7 @@ int mcamd_flash_attn_with_kvcache_ex(const void *q, const void *k, const void *v
  * GPU: calls that overlap on one GPU race. Sizes whose decode partials need more scratch than that
  * (mcamd_attn_workspace_bytes() > MCAMD_NOALLOC_SCRATCH_BYTES) return MCAMD_EWORKSPACE. The
  * stream's device must be the current device. Otherwise identical to
- * mcamd_flash_attn_with_kvcache, with the same kernels and bit-identical results (for t_new > 1,
- * to that call without a workspace).
+ * mcamd_flash_attn_with_kvcache, with the same kernels and bit-identical results.
  */
 #define MCAMD_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
 int mcamd_flash_attn_with_kvcache_noalloc(const void *q, const void *k, const void *v,

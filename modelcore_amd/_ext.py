@@ -46,6 +46,9 @@ SIGNATURES = {
     "mcamd_flash_attn_with_kvcache_ex": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64,
                                                 _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int,
                                                 _int, ctypes.c_int32, _i64, _ptr, _size, _ptr]),
+    "mcamd_flash_attn_with_kvcache_scratch": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64,
+                                                     _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int,
+                                                     _int, ctypes.c_int32, _i64, _ptr, _size, _ptr]),
     "mcamd_flash_attn_with_kvcache_noalloc": (_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                                      _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                                      _i64, _int, _int, _ptr]),

@@ -121,13 +121,14 @@ namespace {
 
 // The cached-attention operator: append, then decode (t_new == 1) or chunked prefill; with
 // `advance` != 0 the positions then move on by that much (the decode step's cache advance);
-// `shared_prefix` > 0 states that keys [0, shared_prefix) are the same in every row.
+// `shared_prefix` > 0 states that keys [0, shared_prefix) are the same in every row. `workspace` is
+// used by decode, and by a prefill if `scratch` is set.
 int kvcache_operator(const void *q, const void *k, const void *v, void *k_cache, void *v_cache,
                      const int32_t *cache_seqlens, int32_t *advance_seqlens, int advance,
                      int64_t shared_prefix, void *out, int64_t batch, int64_t t_new,
                      int64_t n_head, int64_t n_kv_head, int64_t head_dim, int64_t t_max,
                      int64_t cache_batch_stride, int64_t window, int dtype, void *workspace,
-                     size_t workspace_bytes, hipStream_t stream) {
+                     size_t workspace_bytes, bool scratch, hipStream_t stream) {
   if ((k == nullptr) != (v == nullptr))
     return fail(MCAMD_EINVAL, "flash_attn_with_kvcache: pass both k and v, or neither");
   AttnArgs a{q,     k,     v,      k_cache, v_cache,  cache_seqlens, out,
@@ -135,6 +136,12 @@ int kvcache_operator(const void *q, const void *k, const void *v, void *k_cache,
              window, dtype, workspace, workspace_bytes, stream};
   int st = check_attn_shapes(a, t_new == 1);
   if (st != MCAMD_OK) return st;
+  if (t_new != 1 && !scratch) {
+    a.workspace = nullptr;
+    a.workspace_bytes = 0;
+  }
+  if (!aligned(a.workspace, 16))
+    return fail(MCAMD_EINVAL, "flash_attn_with_kvcache: scratch not 16-byte aligned");
   if (shared_prefix < 0 || shared_prefix > t_max)
     return fail(MCAMD_EINVAL, "flash_attn_with_kvcache: shared_prefix outside [0, t_max]");
   if (batch == 0) {
@@ -211,7 +218,7 @@ extern "C" int mcamd_flash_attn_with_kvcache(const void *q, const void *k, const
   (void)causal;
   return kvcache_operator(q, k, v, k_cache, v_cache, cache_seqlens, nullptr, 0, 0, out, batch,
                           t_new, n_head, n_kv_head, head_dim, t_max, cache_batch_stride, window,
-                          dtype, workspace, workspace_bytes, as_stream(stream));
+                          dtype, workspace, workspace_bytes, false, as_stream(stream));
 }
 
 extern "C" int mcamd_flash_attn_with_kvcache_ex(
@@ -223,6 +230,19 @@ extern "C" int mcamd_flash_attn_with_kvcache_ex(
   (void)causal;
   return kvcache_operator(q, k, v, k_cache, v_cache, cache_seqlens, cache_seqlens, advance,
                           shared_prefix, out, batch, t_new, n_head, n_kv_head, head_dim, t_max,
-                          cache_batch_stride, window, dtype, workspace, workspace_bytes,
+                          cache_batch_stride, window, dtype, workspace, workspace_bytes, false,
+                          as_stream(stream));
+}
+
+extern "C" int mcamd_flash_attn_with_kvcache_scratch(
+    const void *q, const void *k, const void *v, void *k_cache, void *v_cache,
+    int32_t *cache_seqlens, void *out, int64_t batch, int64_t t_new, int64_t n_head,
+    int64_t n_kv_head, int64_t head_dim, int64_t t_max, int64_t cache_batch_stride,
+    int64_t window, int causal, int dtype, int32_t advance, int64_t shared_prefix,
+    void *scratch, size_t scratch_bytes, void *stream) {
+  (void)causal;
+  return kvcache_operator(q, k, v, k_cache, v_cache, cache_seqlens, cache_seqlens, advance,
+                          shared_prefix, out, batch, t_new, n_head, n_kv_head, head_dim, t_max,
+                          cache_batch_stride, window, dtype, scratch, scratch_bytes, true,
                           as_stream(stream));
 }

@@ -214,7 +214,9 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, cache_seqlens=N
             int(bool(causal)), code)
     ws_args = (ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
                _ext.stream_handle(q.device))
-    if advance or shared_prefix:
+    if T_new != 1:
+        st = lib.mcamd_flash_attn_with_kvcache_scratch(*args, advance, shared_prefix, *ws_args)
+    elif advance or shared_prefix:
         st = lib.mcamd_flash_attn_with_kvcache_ex(*args, advance, shared_prefix, *ws_args)
     else:
         st = lib.mcamd_flash_attn_with_kvcache(*args, *ws_args)

@@ -51,6 +51,17 @@ def test_attention_rejects_bad_head_grouping_and_small_workspace():
     assert st == _ext.EINVAL and b"both k and v" in lib.mcamd_last_error()
 
 
+def test_scratch_of_a_multi_token_call_must_be_aligned():
+    lib = _ext.lib()
+    fake = 1 << 20  # never dereferenced: the checks fail first
+    args = (fake, fake, fake, fake, fake, fake, fake, 1, 100, 8, 4, 128, 64, 64 * 4 * 128, -1, 1,
+            _ext.BF16, 0, 0)
+    st = lib.mcamd_flash_attn_with_kvcache_scratch(*args, fake + 8, 1 << 30, None)
+    assert st == _ext.EINVAL and b"aligned" in lib.mcamd_last_error()
+    st = lib.mcamd_flash_attn_with_kvcache_scratch(*args[:8], 1, *args[9:], fake, 16, None)
+    assert st == _ext.EWORKSPACE  # one token: the workspace it always needed
+
+
 def test_workspace_size_follows_the_split_count():
     lib = _ext.lib()
     B, H, D, T_max = 32, 16, 128, 8300

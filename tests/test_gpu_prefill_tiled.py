@@ -178,6 +178,47 @@ def test_key_ranges_with_rows_outside_the_cache_and_non_finite_values(dtype, D):
         assert torch.isfinite(out[1, :, :2, :3]).all() and torch.isfinite(out[1, :, :2, 4:]).all()
 
 
+def _c_entry(g, dtype, ws, scratch_entry):
+    """The C operator on copies of the case's caches; returns its output."""
+    B, T_new, H, D = g["q"].shape
+    T_max, H_kv = g["k_cache"].shape[1:3]
+    kc, vc, out = g["k_cache"].clone(), g["v_cache"].clone(), torch.empty_like(g["q"])
+    args = (g["q"].data_ptr(), g["k"].data_ptr(), g["v"].data_ptr(), kc.data_ptr(), vc.data_ptr(),
+            g["cache_seqlens"].data_ptr(), out.data_ptr(), B, T_new, H, H_kv, D, T_max, kc.stride(0),
+            -1, 1, _ext.dtype_code(dtype))
+    tail = (ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
+            _ext.stream_handle(DEV))
+    lib = _ext.lib()
+    if scratch_entry:
+        st = lib.mcamd_flash_attn_with_kvcache_scratch(*args, 0, 0, *tail)
+    else:
+        st = lib.mcamd_flash_attn_with_kvcache(*args, *tail)
+    _ext.check(st, "C entry")
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 128)])
+def test_the_workspace_of_the_operator_is_left_alone(dtype, D):
+    """mcamd_flash_attn_with_kvcache never touches its workspace in a multi-token call, whatever its
+    size: a caller may share one between streams. Scratch that is too small leaves the keys whole,
+    with the same bits."""
+    print("case: ranges, workspace", dtype, D, flush=True)
+    c = make_case([2000, 31], 20, 8, 2, D, 2100, dtype, seed=45)
+    g = _gpu(c)
+    need = _ext.lib().mcamd_attn_scratch_bytes(2, 20, 8, 2, D, 2100, -1, _ext.dtype_code(dtype))
+    assert need > 0
+    ws = torch.full((2 * need,), 7, dtype=torch.uint8, device=DEV)
+    whole = _c_entry(g, dtype, None, False)
+    assert torch.equal(_c_entry(g, dtype, ws, False), whole)
+    assert (ws == 7).all()
+    assert torch.equal(_c_entry(g, dtype, ws[:need - 16], True), whole)
+    assert (ws == 7).all()
+    cut = _c_entry(g, dtype, ws, True)
+    assert not (ws == 7).all()
+    assert torch.equal(cut, _run(c, -1))
+
+
 def test_without_scratch_the_keys_stay_whole():
     """The C entry without a workspace gives the same call within its rounding, and the same bits
     whatever stream it runs on."""
