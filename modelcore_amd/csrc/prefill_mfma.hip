@@ -227,6 +227,7 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
   const int p_last = s0 + q_end - 1;
   int lo = P.window >= 0 ? max(0, p_first - P.window) : 0;
   int hi = p_last;
+  const int lo_block = lo;
   bool whole = true;
   if constexpr (SPLIT) {  // this workgroup's range of the block's tiles
     const int tiles = (hi - lo) / KT + 1;
@@ -393,10 +394,32 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
   // measured 4.4% slower (1011-1013 against 1056-1058 TFLOP/s, two paired runs).
   const int n_tiles = (hi - lo) / KT + 1;
   const int lag = wave >= 4 ? 1 : 0;
-  issue_tile(lo, 0);
-  if (n_tiles > 1) issue_tile(lo + KT, 1);
   f32x16 sc[2];
   bf16x8 pk[4];
+  const bool later = SPLIT && part > 0;
+  if (later) {  // the block's first keys, into the buffer that is taken last
+    issue_part(lo_block, 3, 0);
+    issue_part(lo_block, 3, 2);
+  }
+  issue_tile(lo, 0);
+  if (n_tiles > 1) issue_tile(lo + KT, 1);
+  if (later) {
+    // A later range starts from the maximum over the block's first tile, as the whole block's walk
+    // does: its weights are then rounded to bf16 as they are there, and the ranges differ from the walk
+    // by the order of the fp32 sums alone. (Against each range's own first tile, 100 tokens after 8000
+    // keys differed by 3.0e-3 of the output's norm, with the same error against 64 bits.)
+    if (n_tiles > 1)
+      __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): both tiles after it may be pending
+    else
+      __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4)
+    __builtin_amdgcn_s_barrier();
+    scores(sc, sK[3]);
+    mask(sc, lo_block);
+    m = tile_max(sc);
+    const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) negm[e] = -m_use;
+  }
   for (int slot = 0; slot < 2 * n_tiles + 2; ++slot) {
     if ((slot & 1) == 0) {
       // Tile slot / 2 has landed once only the four DMAs of tile slot / 2 + 1 may be pending.

@@ -219,6 +219,24 @@ def test_the_workspace_of_the_operator_is_left_alone(dtype, D):
     assert torch.equal(cut, _run(c, -1))
 
 
+@pytest.mark.parametrize("seqlens,T_new,H,H_kv,T_max", [([8000], 100, 32, 8, 8200), ([1500, 700], 17, 12, 4, 4000)])
+def test_key_ranges_weigh_as_the_whole_walk_does(seqlens, T_new, H, H_kv, T_max):
+    """bf16 weights are rounded against the maximum of a block's first tile, in every range of it, so
+    cut and whole calls differ by the order of fp32 sums alone, where that moves the output's own
+    rounding: by 2^-8 of a value in a few of a thousand, 2e-4 of the norm at most. Weights rounded
+    against another maximum differ by about 2^-9 / sqrt(3) each way, 2e-3."""
+    dtype, D = torch.bfloat16, 128
+    print("case: ranges, weights", seqlens, T_new, H, H_kv, T_max, flush=True)
+    c = make_case(seqlens, T_new, H, H_kv, D, T_max, dtype, seed=48)
+    c["k_cache"] *= 1.2
+    g = _gpu(c)
+    need = _ext.lib().mcamd_attn_scratch_bytes(len(seqlens), T_new, H, H_kv, D, T_max, -1, _ext.BF16)
+    assert need > 0
+    whole = to_np(_c_entry(g, dtype, None, True))
+    cut = to_np(_c_entry(g, dtype, torch.empty(need, dtype=torch.uint8, device=DEV), True))
+    assert np.linalg.norm(cut - whole) <= 2e-4 * np.linalg.norm(whole)
+
+
 def test_without_scratch_the_keys_stay_whole():
     """The C entry without a workspace gives the same call within its rounding, and the same bits
     whatever stream it runs on."""
