@@ -155,13 +155,13 @@ int kvcache_operator(const void *q, const void *k, const void *v, void *k_cache,
     a.shared_prefix = shared_prefix;
     return launch_decode(a);
   }
-  if (k) {
+  if (k && !prefill_appends(a)) {
     AppendArgs ap{k,       v,        k_cache, v_cache, cache_seqlens,      batch, t_new,
                   n_kv_head, head_dim, t_max, cache_batch_stride, dtype, stream};
     st = launch_append(ap);
     if (st != MCAMD_OK) return st;
+    a.k_new = a.v_new = nullptr;
   }
-  a.k_new = a.v_new = nullptr;
   st = launch_prefill(a);
   if (st != MCAMD_OK) return st;
   return launch_advance(advance_seqlens, batch, advance, stream);

@@ -29,8 +29,9 @@ int launch_advance_varlen(int32_t *seqlens, const int32_t *rows, const int32_t *
 
 struct AttnArgs {
   const void *q;
-  const void *k_new, *v_new;  // decode only: the token at position cache_seqlens[b] is read from
-                              // here instead of the cache (NULL = read it from the cache)
+  const void *k_new, *v_new;  // decode, and where prefill_appends(): the tokens from position
+                              // cache_seqlens[b] on are read from here instead of the cache and
+                              // stored there (NULL = they are in the cache)
   const void *k_cache, *v_cache;
   const int32_t *seqlens;
   void *out;
@@ -114,6 +115,11 @@ int launch_prefill_tiled(const AttnArgs &a);
 
 // The bf16 / head_dim 128 chunked prefill on the matrix cores.
 bool prefill_mfma_supported(const AttnArgs &a);
+// Whether a call with these arguments appends k_new and v_new itself (else they are appended first and
+// not given): the calls whose keys are cut into ranges. They read the chunk's keys from k_new and
+// v_new, and the merge, which they launch in any case, stores them, so that they take no launch more
+// than uncut ones.
+bool prefill_appends(const AttnArgs &a);
 int launch_prefill_mfma(const AttnArgs &a);
 // Key ranges of these calls (prefill_split.h), and the merge of their partials into the output;
 // careful: results that are not finite are redone key by key.

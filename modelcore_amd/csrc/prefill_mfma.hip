@@ -146,19 +146,24 @@ __device__ __forceinline__ float exp2_or_zero(float x) {
   return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x);
 }
 
-// SPLIT: a workgroup per key range of a block (prefill_split.h). VARLEN: sequences of their own
+// SPLIT: a workgroup per key range of a block (prefill_split.h), which takes the chunk's own keys from
+// k_new and v_new where they are given (the merge appends them). VARLEN: sequences of their own
 // lengths, packed along the token axis.
 template <bool SPLIT, bool VARLEN>
-__device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const SplitGeo *S) {
+__device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const SplitGeo *S,
+                                                  const uint16_t *k_new, const uint16_t *v_new) {
   __shared__ __attribute__((aligned(1024))) uint16_t sK[4][TILE];
   __shared__ __attribute__((aligned(1024))) uint16_t sV[4][TILE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   int bh = blockIdx.x % P.n_bh;
-  const int rest = blockIdx.x / P.n_bh;
-  const int part = SPLIT ? rest % S->n_split : 0;  // key range
-  int qt = SPLIT ? rest / S->n_split : rest;
+  int qt = blockIdx.x / P.n_bh;
+  int part = 0;  // key range: every block's first, which are there whether or not it is cut, then the rest
+  if constexpr (SPLIT) {
+    part = qt / P.n_qt;
+    qt -= part * P.n_qt;
+  }
   // The longest blocks, a prompt's last, first (two prompts of 4096 tokens, 12 / 4 heads: 147 us in
   // the other order, 118 so). With a window most are alike, and ascending they share its keys in
   // L2 (eight of 2048 tokens, window 1024: 113 us, 115 descending); blocks that all start at once
@@ -259,8 +264,26 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
   const uint32_t v_chunk = uint32_t((lane & 15) ^ (4 * ((lane >> 4) & 3)));
   // Part i (0..3) of this wave's share of a tile: K fragment 2w + i / 2 (i even) or V block
   // 2w + i / 2 (i odd).
+  // SPLIT: key `key` of the cache, or of the chunk from position s0 on.
+  const int64_t new_at = (tok0 * P.H_kv + kvh) * D;
+  auto key_at = [&](const uint16_t *cached, const uint16_t *fresh, int key) {
+    const bool is_new = fresh != nullptr && key >= s0;
+    const char *base = reinterpret_cast<const char *>(is_new ? fresh + new_at : cached);
+    return base + __umul24(uint32_t(is_new ? key - s0 : key), tok_bytes);
+  };
   auto issue_part = [&](int k0, int buf, int i) {
     const int f = 2 * wave_s + (i >> 1);
+    if constexpr (SPLIT) {
+      const bool is_k = (i & 1) == 0;
+      const int key = min(k0 + (is_k ? 32 * (f >> 3) + col : 4 * f + (lane >> 4)), hi);
+      const char *at = is_k ? key_at(kbase, k_new, key) + 32 * (f & 7) + k_lane_off
+                            : key_at(vbase, v_new, key) + ((v_chunk ^ uint32_t(f & 3)) << 4);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void *)(at),
+          (__attribute__((address_space(3))) void *)(is_k ? &sK[buf][f * 512] : &sV[buf][f * 512]),
+          16, 0, 0);
+      return;
+    }
     if ((i & 1) == 0) {
       const uint32_t kkey = uint32_t(min(k0 + 32 * (f >> 3) + col, hi));
       const uint32_t off = __umul24(kkey, tok_bytes) + uint32_t(16 * (f & 7)) * 2u + k_lane_off;
@@ -482,6 +505,9 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
       l += tl;
     } else {
       const int t = ph / 2 - 1;  // M(t)
+      // SPLIT: all parts before the fragments are live (their 64-bit addresses take registers).
+      if constexpr (SPLIT)
+        for (int i = 0; i < 4; ++i) dma_part(i);
       // The matrix phase at raised wave priority: when the matrix core frees, the SIMD issues
       // this wave's next product before its partner's VALU work (measured: +1.4-2.3% on the 16K
       // chunked prefill; the opposite preference costs 7%).
@@ -530,7 +556,7 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
           pair(ks_c, std::integral_constant<int, 1>{});
           pair(ks_c, std::integral_constant<int, 2>{});
           pair(ks_c, std::integral_constant<int, 3>{});
-          dma_part(ks);
+          if constexpr (!SPLIT) dma_part(ks);
         };
         auto issue = [&](auto ks_c, int buf) {
           issue_i(ks_c, std::integral_constant<int, 0>{}, buf);
@@ -547,7 +573,7 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           pv_step(pk[ks], ks, sV[t % 4]);
-          dma_part(ks);
+          if constexpr (!SPLIT) dma_part(ks);
         }
       }
       __builtin_amdgcn_s_setprio(0);
@@ -588,13 +614,14 @@ __device__ __forceinline__ void prefill_mfma_body(const MfmaParams &P, const Spl
 }
 
 __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(MfmaParams P) {
-  prefill_mfma_body<false, false>(P, nullptr);
+  prefill_mfma_body<false, false>(P, nullptr, nullptr, nullptr);
 }
 __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_varlen_kernel(MfmaParams P) {
-  prefill_mfma_body<false, true>(P, nullptr);
+  prefill_mfma_body<false, true>(P, nullptr, nullptr, nullptr);
 }
-__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_split_kernel(MfmaParams P, SplitGeo S) {
-  prefill_mfma_body<true, false>(P, &S);
+__global__ __launch_bounds__(kThreads, 1) void prefill_mfma_split_kernel(
+    MfmaParams P, SplitGeo S, const uint16_t *k_new, const uint16_t *v_new) {
+  prefill_mfma_body<true, false>(P, &S, k_new, v_new);
 }
 
 }  // namespace
@@ -621,6 +648,10 @@ SplitPlan prefill_mfma_plan(const AttnArgs &a) {
   plan_splits(a, device_cus(), 1.4f,
               a.window >= 0 ? std::min<int64_t>(a.t_max, a.window + QT) : a.t_max, p);
   return p;
+}
+
+bool prefill_appends(const AttnArgs &a) {
+  return prefill_mfma_supported(a) && a.batch > 0 && split_geo(a, prefill_mfma_plan(a)).n_split > 1;
 }
 
 int launch_prefill_mfma(const AttnArgs &a) {
@@ -659,7 +690,8 @@ int launch_prefill_mfma(const AttnArgs &a) {
     return launch_status("prefill_mfma");
   }
   hipLaunchKernelGGL(prefill_mfma_split_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, a.stream,
-                     P, geo);
+                     P, geo, static_cast<const uint16_t *>(a.k_new),
+                     static_cast<const uint16_t *>(a.v_new));
   const int st = launch_status("prefill_mfma");
   if (st != MCAMD_OK) return st;
   return launch_prefill_combine(a, geo, false);

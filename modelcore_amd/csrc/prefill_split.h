@@ -15,10 +15,18 @@
 // by 32 dims in 4 x 64 lanes of four dims (lane (h, col) of step j: pair col, dims 8j + 4h ..), so
 // that every access of a wave is 1 KiB in one piece.
 //
+// Where nothing is cut (a first prompt in a long cache: the host sees the same sizes), the second
+// launch is not to cost more than it saves elsewhere: on the bf16 / 128 path it appends the chunk, whose
+// keys the ranges read from k and v, and so takes the place of the append's launch; the first ranges of
+// all blocks are launched first; and rows too short for a cut are known by one comparison
+// (uncut_keys). 100 tokens from position 0 of a 16384-key cache, 32 / 8 heads of 128: 13.0 us with the
+// append (15.7 with an append of its own and every workgroup working out its ranges; 12.6 without
+// scratch); 500 tokens 24.9 (31.8; 23.9).
+//
 // Measured (100 tokens of 32 query / 8 KV heads of 128 in bf16 after 8000 keys; 16 blocks of 126
-// tiles, the attention without its append): uncut 180 us; cut 38 us, of which the merge 9. With
-// partials as rows of D floats (16 bytes of each of 32 rows per store) 44, with the merge's loads
-// one range at a time 42. The partials' rate was swept: 2e6 44 us, 4e6 40, 6e6 38, 9e6 36.7; from
+// tiles): uncut 182 us; cut 36.3, of which the merge, with the append, 9.3. With
+// partials as rows of D floats (16 bytes of each of 32 rows per store) 6 us more, with the merge's loads
+// one range at a time 4. The partials' rate was swept: 2e6 44 us, 4e6 40, 6e6 38, 9e6 36.7; from
 // 9e6 on, calls of many rows and few keys lose to the uncut ones (8 x 20 tokens after 500 keys: 28.7
 // against 21.0 us).
 #pragma once
@@ -44,6 +52,7 @@ struct SplitGeo {
   int groups;      // 32-pair groups per block
   int md;          // 32-dim pieces of the head
   int G, window;
+  int uncut_keys;  // rows of at most that many keys are not cut, whatever the block
   float ratio;     // tile time / time of one range's partials of the whole call
   float *part_o;   // [n_split][n_qt * n_bh * groups][md][4][64][4]
   float *part_ml;  // [n_split][n_qt * n_bh * groups][32][2]
@@ -78,6 +87,7 @@ __host__ __device__ inline int best_splits(float ratio, int tiles, int kt, int m
 
 // Ranges of a block of n_tiles tiles.
 __device__ __forceinline__ int block_splits(const SplitGeo &g, int s0, int T_b, int n_tiles) {
+  if (s0 + T_b <= g.uncut_keys) return 1;
   int lo, hi;
   block_keys(g, s0, T_b, int((int64_t(T_b) * g.G - 1) / g.pairs), lo, hi);
   const int longest = max((hi - lo) / g.kt + 1, n_tiles);
@@ -132,6 +142,12 @@ inline SplitGeo split_geo(const AttnArgs &a, const SplitPlan &p) {
   g.G = int(a.n_head / a.n_kv_head);
   g.window = int(a.window < 0 ? -1 : a.window);
   g.ratio = p.ratio;
+  g.uncut_keys = 0;
+  if (g.n_split > 1) {  // one tile less than would be cut: the device's roots need not be the host's
+    int tiles = 1;
+    while (best_splits(p.ratio, tiles, p.kt, g.n_split) < 2) ++tiles;
+    g.uncut_keys = (tiles - 2) * p.kt;
+  }
   g.part_o = static_cast<float *>(a.workspace);
   g.part_ml = g.part_o + size_t(g.n_split) * p.blocks * g.groups * g.md * 1024;
   return g;

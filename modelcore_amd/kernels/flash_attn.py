@@ -22,6 +22,7 @@ so code and tests that set them keep working; they select nothing here.
 """
 from __future__ import annotations
 
+import functools
 import os
 from types import SimpleNamespace
 
@@ -127,6 +128,12 @@ def _check_seqlens(cache_seqlens, B, device):
     return cache_seqlens.contiguous()
 
 
+@functools.lru_cache(maxsize=1024)
+def _scratch_bytes(device_index, *sizes):
+    """mcamd_attn_scratch_bytes, a function of the sizes and the device alone: 0.06 us against 0.65."""
+    return _ext.lib().mcamd_attn_scratch_bytes(*sizes)
+
+
 def _window(window_size):
     w = int(window_size[0])
     return -1 if w < 0 else w
@@ -206,7 +213,7 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, cache_seqlens=N
         ws = _ext.workspace(q.device, lib.mcamd_attn_workspace_bytes(B, 1, H, H_kv, D, T_max, w))
     else:
         # Scratch of the call's own: prefills on several streams share nothing.
-        ws_bytes = lib.mcamd_attn_scratch_bytes(B, T_new, H, H_kv, D, T_max, w, code)
+        ws_bytes = _scratch_bytes(q.device.index, B, T_new, H, H_kv, D, T_max, w, code)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     args = (q.data_ptr(), k.data_ptr() if k is not None else None,
             v.data_ptr() if v is not None else None, k_cache.data_ptr(), v_cache.data_ptr(),

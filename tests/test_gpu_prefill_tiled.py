@@ -178,6 +178,38 @@ def test_key_ranges_with_rows_outside_the_cache_and_non_finite_values(dtype, D):
         assert torch.isfinite(out[1, :, :2, :3]).all() and torch.isfinite(out[1, :, :2, 4:]).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("seqlens,T_new,H,H_kv,D,T_max,window", [
+    ([1990, 1200, -1, -20, 0, 2003], 33, 4, 2, 128, 2000, -1),   # rows partly and wholly outside
+    ([700, 0, 63], 130, 6, 3, 128, 1100, 400),
+    ([2500], 2, 32, 8, 128, 2502, -1),                           # the cache's last positions
+    ([900, 5], 40, 4, 2, 96, 2000, -1),
+])
+def test_calls_with_key_ranges_append_bit_for_bit(dtype, seqlens, T_new, H, H_kv, D, T_max, window):
+    print("case: ranges, append", dtype, seqlens, T_new, H, H_kv, D, T_max, window, flush=True)
+    c = make_case([max(0, min(s, T_max - T_new)) for s in seqlens], T_new, H, H_kv, D, T_max, dtype,
+                  seed=47)
+    ok = [i for i, s in enumerate(seqlens) if 0 <= s <= T_max - T_new]
+    ref = _oracle(c, window)
+    c["cache_seqlens"] = torch.tensor(seqlens, dtype=torch.int32)
+    assert _ext.lib().mcamd_attn_scratch_bytes(len(seqlens), T_new, H, H_kv, D, T_max, window,
+                                               _ext.dtype_code(dtype)) > 0
+    g = _gpu(c)
+    out = flash_attn.flash_attn_with_kvcache(g["q"], g["k_cache"], g["v_cache"], k=g["k"], v=g["v"],
+                                             cache_seqlens=g["cache_seqlens"], causal=True,
+                                             window_size=(window, 0))
+    assert np.abs(to_np(out[ok]) - ref[ok]).max() <= ATOL[dtype]
+    assert torch.isnan(out[[i for i in range(len(seqlens)) if i not in ok]]).all()
+    want = {n: c[n].clone() for n in ("k_cache", "v_cache")}
+    for b, s in enumerate(seqlens):
+        for t in range(T_new):
+            if 0 <= s + t < T_max:
+                want["k_cache"][b, s + t] = c["k"][b, t]
+                want["v_cache"][b, s + t] = c["v"][b, t]
+    for n in want:
+        assert torch.equal(g[n].cpu(), want[n]), n
+
+
 def _c_entry(g, dtype, ws, scratch_entry):
     """The C operator on copies of the case's caches; returns its output."""
     B, T_new, H, D = g["q"].shape
