@@ -1,9 +1,10 @@
 """The matrix-core chunked prefill for fp32 caches and head dims other than 128
-(prefill_tiled.hip), and the key ranges of calls with few query blocks (prefill_split.h), at the edges of its tiles: 32 and 128 pairs per workgroup, 32, 64 and 128
-keys per tile, every head-dim instantiation with and without padded dims.
+(prefill_tiled.hip), and the key ranges of calls with few query blocks (prefill_split.h), at the
+edges of its tiles: 32 and 128 pairs per workgroup, 32, 64 and 128 keys per tile, every head-dim
+instantiation with and without padded dims.
 
-Tolerance: bf16 rounds the output once (at most 2^-8 of it: 8 bits) and holds the weights to 2^-17, so the sums
-are within 2^-17 * max|v| < 5e-5 plus fp32 summation: 1e-4. fp32: 2e-5, as for every kernel.
+Tolerance: bf16 rounds the output once (at most 2^-8 of it: 8 bits) and holds the weights to 2^-17, so
+the sums are within 2^-17 * max|v| < 5e-5 plus fp32 summation: 1e-4. fp32: 2e-5, as for every kernel.
 """
 import numpy as np
 import pytest
@@ -270,8 +271,7 @@ def test_key_ranges_weigh_as_the_whole_walk_does(seqlens, T_new, H, H_kv, T_max)
 
 
 def test_without_scratch_the_keys_stay_whole():
-    """The C entry without a workspace gives the same call within its rounding, and the same bits
-    whatever stream it runs on."""
+    """The C entry without a workspace gives the same call within its rounding."""
     print("case: ranges, no scratch", flush=True)
     c = make_case([2000, 31], 20, 8, 2, 64, 2100, torch.float32, seed=45)
     out = _run(c, -1)
@@ -284,3 +284,91 @@ def test_without_scratch_the_keys_stay_whole():
     _ext.check(st, "no scratch")
     _close(whole, _oracle(c, -1), torch.float32)
     _close(out, _oracle(c, -1), torch.float32)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 128)])
+def test_key_ranges_on_two_streams_and_captured(dtype, D):
+    """Each call has scratch of its own: calls that overlap on two streams, and a captured one replayed
+    between other calls, give the bits of calls by themselves."""
+    print("case: ranges, streams", dtype, D, flush=True)
+    T_new, H, H_kv, T_max = 20, 8, 2, 2100
+    cases = [_gpu(make_case(s, T_new, H, H_kv, D, T_max, dtype, seed=49 + i))
+             for i, s in enumerate(([2000, 31], [900, 1700]))]
+    assert _ext.lib().mcamd_attn_scratch_bytes(2, T_new, H, H_kv, D, T_max, -1,
+                                               _ext.dtype_code(dtype)) > 0
+
+    def call(g):
+        return flash_attn.flash_attn_with_kvcache(g["q"], g["k_cache"], g["v_cache"], k=g["k"],
+                                                  v=g["v"], cache_seqlens=g["cache_seqlens"],
+                                                  causal=True)
+
+    want = [call(g) for g in cases]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = [[], []]
+    for _ in range(5):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(call(cases[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for y in got[i]:
+            assert torch.equal(y, want[i])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = call(cases[0])
+    for _ in range(3):
+        y.fill_(float("nan"))
+        cases[0]["k_cache"][0, 2000:2000 + T_new] = 0  # the replay appends again
+        assert torch.equal(call(cases[1]), want[1])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[0])
+        assert torch.equal(cases[0]["k_cache"][0, 2000:2000 + T_new], cases[0]["k"][0])
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("rows,T_new,pos,H,H_kv", [(8, 512, 0, 12, 12), (12, 40, 1500, 8, 2), (60, 1, 900, 12, 12)],
+                         ids=["prompts", "chunks", "decode"])
+def test_a_batch_gives_its_rows_what_they_get_alone(dtype, D, rows, T_new, pos, H, H_kv):
+    """How a call is cut depends on its batch (waves over keys or pairs, key ranges, split length), so
+    not bit for bit: within the rounding of the two."""
+    print("case: batched and alone", dtype, D, rows, T_new, pos, H, H_kv, flush=True)
+    T_max = pos + T_new + 50
+    seqlens = [max(0, pos - 13 * b) for b in range(rows)]
+    c = make_case(seqlens, T_new, H, H_kv, D, T_max, dtype, seed=50)
+    out = to_np(_run(c, -1))
+    for b in (0, rows - 1):
+        alone = to_np(_run({n: t[b:b + 1].contiguous() for n, t in c.items()}, -1))
+        err = np.abs(out[b:b + 1] - alone)
+        if dtype == torch.float32:
+            assert err.max() <= 2 * ATOL[dtype]
+        elif D == 64:
+            assert np.all(err <= np.abs(alone) * 2.0 ** -7 + 2e-4)
+        else:
+            assert err.max() <= ATOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 64), (torch.bfloat16, 128)])
+def test_a_long_prompt_in_chunks_is_the_prompt_in_one(dtype, D):
+    """Past 512 keys chunks are cut into ranges, and their tiles start elsewhere than the prompt's
+    blocks: the sums are the same in another order."""
+    print("case: chunks of a long prompt", dtype, D, flush=True)
+    T, C, H, H_kv = 1536, 128, 8, 4
+    c = _gpu(make_case([0], T, H, H_kv, D, T, dtype, seed=52))
+    whole = flash_attn.flash_attn_with_kvcache(c["q"], c["k_cache"], c["v_cache"], k=c["k"], v=c["v"],
+                                               cache_seqlens=c["cache_seqlens"], causal=True)
+    kc, vc = torch.zeros_like(c["k_cache"]), torch.zeros_like(c["v_cache"])
+    pos, parts = c["cache_seqlens"].clone(), []
+    for a in range(0, T, C):
+        parts.append(flash_attn.flash_attn_with_kvcache(
+            c["q"][:, a:a + C], kc, vc, k=c["k"][:, a:a + C], v=c["v"][:, a:a + C], cache_seqlens=pos,
+            causal=True, advance=C))
+    assert torch.equal(kc, c["k_cache"]) and torch.equal(vc, c["v_cache"]) and int(pos) == T
+    got, ref = to_np(torch.cat(parts, 1)), to_np(whole)
+    if dtype == torch.float32:
+        assert np.abs(got - ref).max() <= 2 * ATOL[dtype]
+    elif D == 64:
+        assert np.all(np.abs(got - ref) <= np.abs(ref) * 2.0 ** -7 + 2e-4)
+    else:
+        assert np.abs(got - ref).max() <= ATOL[dtype]
