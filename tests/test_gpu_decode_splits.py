@@ -40,6 +40,7 @@ CASES = [
     ([500, 1], 16, 1, 256, 600, 300),                        # G = 16: two head chunks append once
     ([31, 32, 33], 3, 3, 16, 40, -1),
     ([90, 10], 4, 4, 8, 100, -1),                            # half of each key's two lanes
+    ([(7 * i) % 400 for i in range(260)], 8, 8, 8, 400, -1),  # 2080 workgroups of up to 512 keys
     # 64 rows of four splits each at most, most of them shorter
     ([(37 * i) % 1024 for i in range(64)], 16, 16, 16, 1024, -1),
     ([1023] + [i % 5 for i in range(63)], 32, 16, 16, 1024, -1),

@@ -51,6 +51,12 @@ def test_rows_shorter_than_their_cache_keep_their_decode_workgroups(tmp_path):
         assert n <= 256 or b * h * -(-(span // 8) // n) >= 256, (b, h, d, t, w, e, n)
 
 
+def test_short_caches_of_many_rows_are_not_cut(tmp_path):
+    cases = [(b, h, 64, t, -1, 2) for b, h, t in ((300, 8, 512), (300, 8, 257), (255, 8, 512), (300, 8, 513),
+                                                  (300, 8, 256))]
+    assert _split_lens(tmp_path, cases) == [512, 512, 256, 256, 256]
+
+
 @pytest.mark.parametrize("t_max", [(1 << 24) + 1, 135_000_000, 1 << 30])
 def test_decode_splits_fit_a_grid(tmp_path, t_max):
     cases = [(b, h, 8, t_max, -1, e) for b in (1, 5, 64) for h in (1, 8) for e in (2, 4)]
