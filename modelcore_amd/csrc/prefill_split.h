@@ -6,10 +6,11 @@
 // launches work it out from cache_seqlens. S ranges take a block's n tiles from n * tile time to
 // n / S of it and cost S times the writing and reading of the call's partials, so the best S is
 // sqrt(n * tile time / partial time). The host gives that ratio and the most ranges for which the
-// chip has room (no range is much shorter than kMinRangeKeys keys: short prompts are never cut, so
-// feeding one in chunks gives the bits of feeding it whole); ranges are as long as is best for the block of the row with the most tiles (the
-// one with its last queries), blocks with fewer tiles get fewer of them, and one that is not cut
-// writes its output itself.
+// chip has room. No range is much shorter than kMinRangeKeys keys, so blocks of fewer than twice as many
+// are never cut. Ranges are as long as is best for the block of the row with the most tiles (the one with
+// its last queries), blocks with fewer tiles get fewer of them, and one that is not cut writes its output
+// itself. A cut call's sums run in another order than an uncut one's: the same outputs within the
+// dtype's rounding, not the same bits.
 //
 // A partial is laid out as the accumulators hold it, which is also how the merge reads it: 32 pairs
 // by 32 dims in 4 x 64 lanes of four dims (lane (h, col) of step j: pair col, dims 8j + 4h ..), so
@@ -96,8 +97,8 @@ __device__ __forceinline__ int block_splits(const SplitGeo &g, int s0, int T_b, 
   return max(1, (n_tiles + range / 2) / range);  // at most s: n_tiles <= longest <= s * range
 }
 
-// What a call's kernel makes of it: its blocks, how many workgroups of it the chip holds
-// (`room`), the time of a tile and the most keys of a block.
+// What a call's kernel makes of it: pairs per block and keys per tile, its blocks, and by
+// plan_splits() the most ranges of one and the ratio of the cost rule.
 struct SplitPlan {
   int pairs, kt;
   int64_t blocks;
@@ -114,6 +115,8 @@ inline int64_t split_floats(const AttnArgs &a, const SplitPlan &p) {
   return p.blocks * (p.pairs + 31) / 32 * 32 * ((a.head_dim + 31) / 32 * 32 + 2);
 }
 
+// room: how many workgroups of the call the chip holds; tile_us: the time of a tile; keys: the most a
+// block can have.
 inline void plan_splits(const AttnArgs &a, int64_t room, float tile_us, int64_t keys,
                         SplitPlan &p) {
   p.n_split = 1;

@@ -28,16 +28,17 @@
 //    the wave, so the weights are its B operand in place; the first takes dims 8c + i and
 //    8c + 4 + i, so that a lane reads its K row as 16-byte vectors.
 //
-// Measured against the VALU kernel this replaced (four lanes a row, an LDS float per FMA): four
-// 2048-token prompts of 12 heads of 64 in bf16 1858 -> 64 us (400 TFLOP/s of the attended pairs;
-// bound by the weights' exponentials and conversions on the VALU), in fp32 262 us (98 of the 154
-// TFLOP/s a large fp32 product reaches); two of 512 tokens in fp32 192 -> 29 us.
+// Measured against the VALU kernel this replaced (four lanes a row, an LDS float per FMA), the call
+// with its append: four 2048-token prompts of 12 heads of 64 in bf16 1868 -> 73 us (355 TFLOP/s of the
+// attended pairs), two of 512 tokens in fp32 194 -> 32.
 //
 // Online softmax per pair in fp32 (exp2 domain): weights are made against the running maximum, and
 // the tile's own maximum is taken (and O rescaled) only when a lane's weights of the tile sum past
 // 2^15 or are not finite, or the pair has no maximum yet.
 //
-// LDS holds one tile; the next is loaded into registers while it is consumed. K rows are padded by
+// LDS holds one tile; the next is loaded while it is consumed, into arrays of which the compiler keeps
+// one in scratch memory in most instantiations (48 to 272 bytes a lane: half a tile's loads are waited
+// for, and stored there, before the products start). K rows are padded by
 // 16 bytes (a 16-lane group reads 16 rows at once: their 16-byte pieces then fall on all banks);
 // bf16 V rows to 16 or 48 banks modulo 64 for the transpose reads (four rows of 64 bytes), fp32 V
 // rows by 32 bytes (the two wave halves read rows four apart).
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
   const E *kbase = static_cast<const E *>(P.k_cache) + int64_t(row) * P.cache_b + int64_t(kvh) * D;
   const E *vbase = static_cast<const E *>(P.v_cache) + int64_t(row) * P.cache_b + int64_t(kvh) * D;
 
-  // The next tile, on its way to LDS: piece c = tid + 256 i is 16 bytes of key c / (DP / VEC).
+  // The next tile, on its way to LDS (see above where it waits): piece c = tid + 256 i is 16 bytes of key c / (DP / VEC).
   // Keys past `hi` re-read key `hi` (they are masked); K's dims past the head_dim are zero, V's
   // re-read the last ones (they reach no output).
   uint4 kr[CH], vr[CH];
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
     for (int i = 0; i < CH; ++i) {
       const int c = tid + kThreads * i;
       const int key = c / (DP / VEC), d = (c % (DP / VEC)) * VEC;
-      // The zeroes go in here and not at the load, which would then be waited for at once.
+      // The zeroes go in here and not at the load, all of which would then be waited for at once.
       *reinterpret_cast<uint4 *>(&sK[key * KSTR + d]) = d < D ? kr[i] : make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4 *>(&sV[key * VSTR + d]) = vr[i];
     }
@@ -706,7 +707,7 @@ TiledPlan tiled_plan(const AttnArgs &a) {
   // Fewer workgroups of 128 pairs than compute units: 32 pairs and a quarter of the keys per wave
   // instead (12 heads of 64: 2 x 512 tokens fp32 33 against 50 us, bf16 15.0 against 18.6; 8 x 512,
   // 384 workgroups: 78 against 67 and 31.6 against 21.8). Head dims above 128 keep KS = 1 (a tile of four waves' keys outgrows the LDS).
-  t.ks = a.head_dim <= 128 && (a.t_new * G + 127) / 128 * n_bh < 256 ? 4 : 1;
+  t.ks = a.head_dim <= 128 && (a.t_new * G + 127) / 128 * n_bh < device_cus() ? 4 : 1;
   p.pairs = 128 / t.ks;
   p.kt = t.ks == 4 ? 128 : bf && a.head_dim <= 128 ? 64 : 32;
   p.blocks = (a.t_new * G + p.pairs - 1) / p.pairs * n_bh;

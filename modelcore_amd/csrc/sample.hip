@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kDrawThreads) void sample_kernel(const float *__res
   const uint32_t k0 = uint32_t(seed), k1 = uint32_t(seed >> 32);
   float best = -INFINITY;
   int best_i = 0x7fffffff;
-  // Lane tid handles groups of four consecutive tokens 4 g .. 4 g + 3, g = tid, tid + 256, ...
+  // Thread tid handles groups of four consecutive tokens 4 g .. 4 g + 3, g = tid, tid + 1024, ...
   for (int g = tid; 4 * g < vocab; g += kDrawThreads) {
     Philox r{0, 0, 0, 0};
     if (!greedy) r = philox4x32_10(uint32_t(g), uint32_t(off), uint32_t(off >> 32), 0u, k0, k1);
