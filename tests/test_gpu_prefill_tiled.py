@@ -110,6 +110,28 @@ def test_infinities_and_nan_reach_only_the_pairs_that_see_them(dtype, heads):
     assert torch.equal(out[3], plain[3])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [8, 40, 64, 96, 136, 192, 256])
+@pytest.mark.parametrize("seqlens,T_new,window", [([0, 60], 70, -1), ([120, 190], 9, 64), ([600, 1100], 20, -1)],
+                         ids=["steps", "window", "ranges"])
+def test_redone_pairs_keep_their_other_values(dtype, D, seqlens, T_new, window):
+    """Pairs that see an infinite value are redone 64 keys a step: at the steps' edges, the dims with
+    the infinity and all the others."""
+    print("case: redone", dtype, D, seqlens, T_new, window, flush=True)
+    c = make_case(seqlens, T_new, 4, 2, D, max(seqlens) + T_new + 3, dtype, seed=51)
+    dims = [1, D - 1]
+    ref = _oracle(c, window)
+    for b, s0 in enumerate(seqlens):  # a value that every query of the row sees
+        at = s0 if window < 0 else s0 + T_new - 1 - window
+        rows = c["v"][b, at - s0] if at >= s0 else c["v_cache"][b, at]
+        rows[0, dims] = float("inf")
+    out = _run(c, window)
+    rest = [d for d in range(D) if d not in dims]
+    assert torch.isposinf(out[:, :, :2][..., dims]).all()
+    _close(out[..., rest], ref[..., rest], dtype)
+    _close(out[:, :, 2:], ref[:, :, 2:], dtype)
+
+
 @pytest.mark.parametrize("seqlens,T_new,H,H_kv,D,T_max", [
     ([40, 3], 40, 2, 2, 64, 100),         # the waves over a block's keys
     ([40, 3], 40, 512, 128, 64, 100),     # over its pairs
