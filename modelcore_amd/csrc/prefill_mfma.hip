@@ -651,7 +651,7 @@ SplitPlan prefill_mfma_plan(const AttnArgs &a) {
 }
 
 bool prefill_appends(const AttnArgs &a) {
-  return prefill_mfma_supported(a) && a.batch > 0 && split_geo(a, prefill_mfma_plan(a)).n_split > 1;
+  return prefill_mfma_supported(a) && a.batch > 0 && cuts_keys(a, prefill_mfma_plan(a));
 }
 
 int launch_prefill_mfma(const AttnArgs &a) {

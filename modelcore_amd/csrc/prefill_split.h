@@ -132,12 +132,17 @@ inline size_t split_bytes(const AttnArgs &a, const SplitPlan &p) {
   return p.n_split <= 1 ? 0 : size_t(p.n_split) * size_t(split_floats(a, p)) * 4;
 }
 
-// The geometry for the kernels; without scratch for the partials the keys stay whole.
+// Whether the call has the scratch to cut its keys; without it they stay whole.
+inline bool cuts_keys(const AttnArgs &a, const SplitPlan &p) {
+  return p.n_split > 1 && a.workspace && a.workspace_bytes >= split_bytes(a, p);
+}
+
+// The geometry for the kernels.
 inline SplitGeo split_geo(const AttnArgs &a, const SplitPlan &p) {
   SplitGeo g;
   g.pairs = p.pairs;
   g.kt = p.kt;
-  g.n_split = a.workspace && a.workspace_bytes >= split_bytes(a, p) ? p.n_split : 1;
+  g.n_split = cuts_keys(a, p) ? p.n_split : 1;
   g.n_bh = int(a.batch * a.n_kv_head);
   g.n_qt = int(p.blocks / g.n_bh);
   g.groups = (p.pairs + 31) / 32;
@@ -147,7 +152,7 @@ inline SplitGeo split_geo(const AttnArgs &a, const SplitPlan &p) {
   g.ratio = p.ratio;
   g.uncut_keys = 0;
   if (g.n_split > 1) {  // one tile less than would be cut: the device's roots need not be the host's
-    int tiles = 1;
+    int tiles = std::max(1, int(4.f / p.ratio) - 1);  // two ranges from sqrt(tiles * ratio) = 2 on
     while (best_splits(p.ratio, tiles, p.kt, g.n_split) < 2) ++tiles;
     g.uncut_keys = (tiles - 2) * p.kt;
   }
