@@ -44,7 +44,7 @@ def test_rows_shorter_than_their_cache_keep_their_decode_workgroups(tmp_path):
              for t in (300, 2048, 8218, 16384, 65536, 131072) for w in (-1, 1500) for e in (2, 4)]
     for (b, h, d, t, w, e), n in zip(cases, _split_lens(tmp_path, cases)):
         span = min(t, w + 1) if w >= 0 else t
-        assert n in (32, 64, 128, 256, 512, 1024, 2048)
+        assert n in (64, 128, 256, 512, 1024, 2048)
         if n > 256:
             assert b * h * -(-span // n) >= 8192, (b, h, d, t, w, e, n)
         # Rows of an eighth of the cache's length: a workgroup per compute unit, or 256 keys each.
