@@ -47,7 +47,6 @@ struct DecodeParams {
   float *part_o;   // [B][H][n_splits][D]
   float *part_ml;  // [B][H][n_splits][2]
   int H, H_kv, G, n_hchunks, T_max, window, n_splits, D, SL;
-  int paired;  // order of the splits and heads in the grid
   int64_t cache_b;
   float scale_log2;
 };
@@ -97,7 +96,8 @@ __device__ __forceinline__ float over_groups(float x, const Op &op) {
 
 // DP is head_dim rounded up to a power of two (at least 16): LPT = DP / VEC lanes cover one key
 // row, and lanes past the real head_dim D hold nothing (they load no data and add zeros).
-template <class E, int DP, int GM>
+// PAIRED: the order of the splits and heads in the grid (run_decode()).
+template <class E, int DP, int GM, bool PAIRED>
 __global__ __launch_bounds__(kThreads) void decode_split_kernel(DecodeParams P) {
   constexpr int VEC = Vec<E>::N;
   constexpr int LPT = DP / VEC;        // lanes per key row
@@ -110,11 +110,9 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(DecodeParams P) 
   __shared__ float s_o[kWaves][GM][DP];
 
   const int b = blockIdx.z;
-  int head = blockIdx.x, split = blockIdx.y;
-  if (P.paired) {  // a split past the last one starts past the row's end
-    head = blockIdx.x >> 1;
-    split = 2 * blockIdx.y + ((blockIdx.x + head + b) & 1);
-  }
+  const int head = PAIRED ? blockIdx.x >> 1 : blockIdx.x;
+  // Paired: a split past the last one starts past the row's end.
+  const int split = PAIRED ? 2 * blockIdx.y + ((blockIdx.x + head + b) & 1) : blockIdx.y;
   const int kvh = head / P.n_hchunks;
   const int hc = head - kvh * P.n_hchunks;
   const int h0 = kvh * P.G + hc * GM;
@@ -353,11 +351,21 @@ __global__ __launch_bounds__(kThreads) void decode_combine_kernel(DecodeParams P
 template <class E, int DP, int GM>
 int run_decode(const DecodeParams &P, int B, hipStream_t stream) {
   // The KV heads of a split are neighbours: together they read whole token rows (16 rows of 12
-  // heads of 64 in bf16: 18.8 us with the splits of a head side by side, 16.7 so). paired: two splits
+  // heads of 64 in bf16: 18.8 us with the splits of a head side by side, 16.7 so). Paired: two splits
   // of a head side by side, then the next head's, the first of the two in turn.
+  //
+  // Rows of 512 bytes or 1 KB of a head, where the workgroups fill the chip several times over, are
+  // paired: with a head beside a head, 16 rows of 8000 keys, 8 heads of 256, run at 5.6 TB/s in fp32 (375
+  // us; paired 330) and 5.7 in bf16 (183; 174). Smaller calls don't gain (3 rows of 11000 keys of it in
+  // bf16 58.2 us, paired 61.0), nor other rows (16 rows of 8000 keys, 8 heads of 192 in fp32, 240 and 251).
   const unsigned heads = P.H_kv * P.n_hchunks, splits = P.n_splits;
-  const dim3 grid = P.paired ? dim3(2 * heads, (splits + 1) / 2, B) : dim3(heads, splits, B);
-  hipLaunchKernelGGL((decode_split_kernel<E, DP, GM>), grid, dim3(kThreads), 0, stream, P);
+  constexpr bool kWide = DP * sizeof(E) >= 512;
+  if (kWide && P.D * sizeof(E) % 512 == 0 && int64_t(B) * P.H_kv * P.n_splits >= 2048)
+    hipLaunchKernelGGL((decode_split_kernel<E, DP, GM, kWide>), dim3(2 * heads, (splits + 1) / 2, B),
+                       dim3(kThreads), 0, stream, P);
+  else
+    hipLaunchKernelGGL((decode_split_kernel<E, DP, GM, false>), dim3(heads, splits, B),
+                       dim3(kThreads), 0, stream, P);
   int st = launch_status("decode_split");
   if (st != MCAMD_OK || P.n_splits == 1) return st;
   hipLaunchKernelGGL(decode_combine_kernel<E>, dim3(P.H, B), dim3(kThreads), 0, stream, P);
@@ -478,11 +486,6 @@ int launch_decode(const AttnArgs &a) {
   P.SL = int(decode_split_len(a.batch, a.n_head, a.n_kv_head, a.head_dim, a.t_max, a.window, elem));
   P.n_splits = int(splits_of(a.t_max, a.window, P.SL));
   P.D = int(a.head_dim);
-  // Rows of 512 bytes or 1 KB of a head, where the workgroups fill the chip several times over: with a
-  // head beside a head, 16 rows of 8000 keys, 8 heads of 256, run at 5.6 TB/s in fp32 (375 us; paired
-  // 330) and 5.7 in bf16 (183; 174). Smaller calls don't gain (3 rows of 11000 keys of it in bf16 58.2 us,
-  // paired 61.0), nor other rows (16 rows of 8000 keys, 8 heads of 192 in fp32, 240 and 251).
-  P.paired = a.head_dim * elem % 512 == 0 && a.batch * a.n_kv_head * P.n_splits >= 2048;
   P.cache_b = a.cache_batch_stride;
   P.scale_log2 = float(kLog2e / std::sqrt(double(a.head_dim)));
   const int64_t floats_o = a.batch * a.n_head * P.n_splits * a.head_dim;
