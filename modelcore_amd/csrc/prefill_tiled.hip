@@ -126,10 +126,10 @@ __device__ __forceinline__ bf16x4 lds_read_tr(const uint16_t *p) {
 // Four prompts of 2048 tokens, 12 heads of 64, with an infinity in one head's first value: 4.7 ms in bf16
 // (a key at a time 28; without the infinity 0.07), in every head's 8.1 in fp32 (38; 0.26). 64 values in
 // flight instead of 32 gave 6% and cost the kernel's other waves their registers.
-template <class E, int DP>
+template <class E, int DP, int LOADS = 32>  // LOADS: values (and 16-byte pieces of keys) in flight
 __device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at, int p, int lane,
                              int d0, int d1) {
-  constexpr int N = (DP + 63) / 64, VEC = Vec<E>::N, U = N == 3 ? 8 : 32 / N;
+  constexpr int N = (DP + 63) / 64, VEC = Vec<E>::N, U = N == 3 ? LOADS / 4 : LOADS / N;
   static_assert(64 % U == 0, "whole batches per step");
   const int D = P.D;
   const E *q = static_cast<const E *>(P.q) + at;
@@ -144,7 +144,7 @@ __device__ void careful_pair(const TiledParams &P, int row, int kvh, int64_t at,
   for (int t0 = key_lo(p, P.window); t0 <= p; t0 += 64) {
     const int t = min(t0 + lane, p);
     float s = 0.f;
-    constexpr int KU = DP / VEC < 8 ? DP / VEC : 8;  // pieces of a key in flight
+    constexpr int KU = DP / VEC < LOADS / 4 ? DP / VEC : LOADS / 4;
     for (int c0 = 0; c0 < D; c0 += KU * VEC) {
       uint4 y[KU];
 #pragma unroll
@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_combine_kernel(TiledPar
     const int c = __builtin_ctz(left);
     const int rlo = __shfl(int(uint64_t(row)), c, 64), rhi = __shfl(int(uint64_t(row) >> 32), c, 64);
     const int64_t r = int64_t((uint64_t(uint32_t(rhi)) << 32) | uint32_t(rlo));
-    careful_pair<E, 256>(P, b, kvh, r * P.D, s0 + __shfl(pos, c, 64), lane, d, min(d + 8, P.D));
+    careful_pair<E, 256, 8>(P, b, kvh, r * P.D, s0 + __shfl(pos, c, 64), lane, d, min(d + 8, P.D));
   }
 }
 
