@@ -497,7 +497,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
                                   o[md][4 * j + 3]});
         }
     }
-    for (uint32_t left = bad; left != 0; left &= left - 1) {
+    for (uint32_t left = bad; __builtin_expect(left != 0, 0); left &= left - 1) {
       const int c = w0 + __builtin_ctz(left);
       careful_pair<E, DP>(P, row, kvh, pair_at(c), s0 + pair_pos(c), lane, 0, D);
     }
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(kThreads) void prefill_tiled_kernel(TiledParams P) 
       }
     }
     for (int x = wave; x < 32; x += kWaves) {
-      if (s_bad[x] == 0) continue;
+      if (__builtin_expect(s_bad[x] == 0, 1)) continue;
       careful_pair<E, DP>(P, row, kvh, pair_at(x), s0 + pair_pos(x), lane, 0, D);
     }
   }
@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_combine_kernel(TiledPar
     const int c = __builtin_ctz(left);
     const int rlo = __shfl(int(uint64_t(row)), c, 64), rhi = __shfl(int(uint64_t(row) >> 32), c, 64);
     const int64_t r = int64_t((uint64_t(uint32_t(rhi)) << 32) | uint32_t(rlo));
-    careful_pair<E, 256, 8>(P, b, kvh, r * P.D, s0 + __shfl(pos, c, 64), lane, d, min(d + 8, P.D));
+    careful_pair<E, 256, 4>(P, b, kvh, r * P.D, s0 + __shfl(pos, c, 64), lane, d, min(d + 8, P.D));
   }
 }
 
